@@ -179,6 +179,24 @@ __global__ __launch_bounds__(64) void value_proj_kernel(const E *__restrict__ o_
     }
 }
 
+// v to columns n .. n + 3 of row b of out [batch][N], those in range
+template <typename E>
+__device__ __forceinline__ void store4(E *__restrict__ out, floatx4 v, int b, int n, int batch, int N)
+{
+    using E4 = typename Vec<E>::v4;
+    if (b >= batch)
+        return;
+    E *o = out + (size_t)b * N + n;
+    if (n + 3 < N && (N & 3) == 0) {
+        *(E4 *)o = E4{(E)v[0], (E)v[1], (E)v[2], (E)v[3]};
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (n + i < N)
+                o[i] = (E)v[i];
+    }
+}
+
 // Output projection:
 //   out[b, n] = sum_k x[b, k] W_O[n, k]      (x = the value projection, [B x K], K = n_h * 128)
 // as its transpose D[n][b] on 16x16x32 MFMAs, W_O rows the A operand and x
@@ -237,7 +255,6 @@ __global__ __launch_bounds__(256) void out_proj_kernel(const E *__restrict__ x, 
                                                        int batch, int K, int N, OutProjGeom geo)
 {
     using E8 = typename Vec<E>::v8;
-    using E4 = typename Vec<E>::v4;
     constexpr int kRowHalves = kChunk;           // one row of a stage
     constexpr int kXOff = kCols * kRowHalves;     // halves: x rows follow the W_O rows
     constexpr int kStage = kXOff + 32 * kRowHalves;
@@ -342,16 +359,8 @@ __global__ __launch_bounds__(256) void out_proj_kernel(const E *__restrict__ x, 
             if (!whole) {
                 // every row and column of the tile, so the sums stay in bounds
                 *(floatx4 *)(part + (size_t)slot * kPartTile + bl * kCols + cl) = v;
-            } else if (b < batch) {
-                E *o = out + (size_t)b * N + n;
-                if (n + 3 < N && (N & 3) == 0) {
-                    *(E4 *)o = E4{(E)v[0], (E)v[1], (E)v[2], (E)v[3]};
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (n + i < N)
-                            o[i] = (E)v[i];
-                }
+            } else {
+                store4(out, v, b, n, batch, N);
             }
         }
         first_piece = false;
@@ -366,7 +375,6 @@ template <typename E>
 __global__ __launch_bounds__(256) void reduce_units_kernel(const float *__restrict__ part, E *__restrict__ out,
                                                            int batch, int N, OutProjGeom geo)
 {
-    using E4 = typename Vec<E>::v4;
     const int quads = (N + 3) / 4;
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (t >= batch * quads)
@@ -393,27 +401,322 @@ __global__ __launch_bounds__(256) void reduce_units_kernel(const float *__restri
         for (int i = 0; i < 8; ++i)
             v += p[i];
     }
-    E *o = out + (size_t)b * N + n;
-    if (n + 3 < N && (N & 3) == 0) {
-        *(E4 *)o = E4{(E)v[0], (E)v[1], (E)v[2], (E)v[3]};
+    store4(out, v, b, n, batch, N);
+}
+
+// Output projection of more than 32 rows (use_wide). The 32-row units above stream W_O
+// once per 32 rows; here a unit is 128 output columns x every row (32 RT of
+// them, at most 256), so that W_O crosses once and x is re-read half as often
+// per byte of it.
+//  * Same stream-K split: the (unit, 64-column K chunk) steps, units
+//    outermost, in equal contiguous ranges, one per workgroup, at most one
+//    workgroup per CU.
+//  * 512 threads: wave w computes columns 32 (w mod 4) .. +31 of rows
+//    16 RT (w / 4) .. + 16 RT - 1 over every K-step, on 16x16x32 MFMAs with
+//    W_O rows the A operand and x rows the B operand.
+//  * A ring stage is the chunk's 128 rows of W_O, then 32 RT rows of x, 128
+//    bytes each, filled by direct global->LDS loads of 8 rows; 16-byte chunk
+//    c of row r sits at c ^ (r / 2 mod 8), which puts the 16 rows of an
+//    operand read on 16 different 16-byte positions of a 256-byte LDS bank
+//    period. The ring is as deep as the LDS allows (6 stages at 64 rows, 3 at
+//    256), one barrier per step: after it every wave has read stage j - 1,
+//    whose slot takes chunk j - 1 + kStages.
+//  * The pieces of a unit shared by workgroups go to fp32 tiles in the
+//    workspace, tile (workgroup g, unit u) at slot g + u, in MFMA accumulator
+//    order (every store and load 1 KB contiguous); reduce_wide_kernel adds
+//    them in workgroup order.
+//  * K (a multiple of 128) has no partial chunk; rows past N or past the
+//    batch re-read the last one and are not stored.
+template <int RT>
+struct Wide {
+    static constexpr int kCols = 128;
+    static constexpr int kRows = 32 * RT;
+    static constexpr int kK = 64;                                     // K per stage
+    static constexpr int kStageBytes = (kCols + kRows) * kK * 2;
+    static constexpr int kFit = 160 * 1024 / kStageBytes;
+    static constexpr int kStages = kFit > 6 ? 6 : kFit;
+    static constexpr int kTile = kCols * kRows;                       // floats of a partial tile
+    static constexpr int kWUnits = 2;                                 // W_O load units per wave and stage
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt_at_most()
+{
+    MLA_WAIT_VMCNT(N);
+}
+
+// waits until at most `stages` (0 .. S) younger stages of U load units are in flight
+template <int U, int S>
+__device__ __forceinline__ void wait_younger(int stages)
+{
+    if constexpr (S > 0) {
+        if (stages >= S) {
+            wait_vmcnt_at_most<U * S>();
+            return;
+        }
+        wait_younger<U, S - 1>(stages);
     } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (n + i < N)
-                o[i] = (E)v[i];
+        wait_vmcnt_at_most<0>();
     }
 }
 
-OutProjGeom out_proj_geom(int batch, int K, int N, int cu_count)
+template <typename E, int RT>
+__global__ __launch_bounds__(512) void out_proj_wide_kernel(const E *__restrict__ x, const E *__restrict__ w,
+                                                            E *__restrict__ out, float *__restrict__ part,
+                                                            int batch, int K, int N, OutProjGeom geo)
+{
+    using T = Wide<RT>;
+    using E8 = typename Vec<E>::v8;
+    constexpr int kXUnits = (RT + 1) / 2;  // x load units of waves 0..3; waves 4..7 have RT / 2
+    __shared__ __attribute__((aligned(1024))) char s_ring[T::kStages * T::kStageBytes];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
+    const int wc = wave & 3, wr = wave >> 2;
+    const int s_first = (int)blockIdx.x * geo.per_wg;
+    const int n_steps = min(geo.steps - s_first, geo.per_wg);
+    const unsigned ring_lds = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char *)s_ring;
+
+    // ---- loads: unit u of a stage's W_O (x) part is its rows 8u .. 8u + 7;
+    // lane -> row 8u + lane / 8, stored position lane mod 8. Wave w issues
+    // units w, w + 8, ...
+    const int lrow = 8 * wave + (lane >> 3);                    // row of the wave's first unit
+    const int lchunk = 16 * ((lane & 7) ^ ((lrow >> 1) & 7));    // (the same for rows 64 further)
+    int i_unit = s_first / geo.chunks, i_c = s_first - i_unit * geo.chunks;  // next (unit, chunk) to issue
+    int off_w[T::kWUnits], off_x[kXUnits];
+    const E *w_base = nullptr, *x_base = nullptr;
+    auto set_unit = [&](int unit) {
+        const int n0 = (unit % geo.n_blocks) * T::kCols, b0 = (unit / geo.n_blocks) * T::kRows;
+        w_base = w + (size_t)n0 * K;
+        x_base = x + (size_t)b0 * K;
+#pragma unroll
+        for (int i = 0; i < T::kWUnits; ++i)
+            off_w[i] = min(lrow + 64 * i, N - 1 - n0) * K * 2 + lchunk;
+#pragma unroll
+        for (int i = 0; i < kXUnits; ++i)
+            off_x[i] = min(lrow + 64 * i, batch - 1 - b0) * K * 2 + lchunk;
+    };
+    set_unit(i_unit);
+    auto issue = [&](int slot) {
+        const unsigned dst = ring_lds + slot * T::kStageBytes + 1024 * wave;
+        const E *wb = w_base + (size_t)i_c * T::kK, *xb = x_base + (size_t)i_c * T::kK;
+#pragma unroll
+        for (int i = 0; i < T::kWUnits; ++i)
+            global_to_lds16_at(wb, off_w[i], dst + 8192 * i);
+#pragma unroll
+        for (int i = 0; i < kXUnits; ++i)
+            if (RT % 2 == 0 || i < kXUnits - 1 || wave < 4)
+                global_to_lds16_at(xb, off_x[i], dst + T::kCols * T::kK * 2 + 8192 * i);
+        if (++i_c == geo.chunks) {
+            i_c = 0;
+            ++i_unit;
+            if (i_unit * geo.chunks < geo.steps)
+                set_unit(i_unit);
+        }
+    };
+    // ---- operands: lane (g, i) reads K 32 kk + 8 g .. +7 of row i of a 16-row group
+    const char *a_lane = s_ring + (32 * wc + l16) * (T::kK * 2);
+    const char *x_lane = s_ring + (T::kCols + 16 * RT * wr + l16) * (T::kK * 2);
+    const int sw = (l16 >> 1) & 7;
+
+    floatx4 acc[2][RT];
+    auto clear = [&]() {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+                acc[nt][r] = floatx4{0.f, 0.f, 0.f, 0.f};
+    };
+    clear();
+    int unit = i_unit, c = i_c, piece_c0 = i_c, slot = 0, i_slot = 0;
+    auto next = [](int s) { return s + 1 == T::kStages ? 0 : s + 1; };
+#pragma unroll
+    for (int j = 0; j < T::kStages - 1; ++j)
+        if (j < n_steps) {
+            issue(i_slot);
+            i_slot = next(i_slot);
+        }
+    for (int j = 0; j < n_steps; ++j) {
+        // this wave's units of chunk j have landed (younger chunks stay in
+        // flight; tile stores issued since are younger than them), then every wave's
+        const int younger = min(T::kStages - 2, n_steps - 1 - j);
+        if (RT % 2 == 0 || wave < 4)
+            wait_younger<T::kWUnits + kXUnits, T::kStages - 2>(younger);
+        else
+            wait_younger<T::kWUnits + RT / 2, T::kStages - 2>(younger);
+        lds_barrier();
+        if (j + T::kStages - 1 < n_steps) {
+            issue(i_slot);
+            i_slot = next(i_slot);
+        }
+        const char *as = a_lane + slot * T::kStageBytes, *xs = x_lane + slot * T::kStageBytes;
+#pragma unroll
+        for (int kk = 0; kk < T::kK / 32; ++kk) {
+            const int ch = 16 * ((4 * kk + g) ^ sw);
+            E8 a[2], xv[RT];
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+                a[nt] = *(const E8 *)(as + 16 * nt * (T::kK * 2) + ch);
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+                xv[r] = *(const E8 *)(xs + 16 * r * (T::kK * 2) + ch);
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt)
+                    acc[nt][r] = mfma16x16x32(a[nt], xv[r], acc[nt][r]);
+        }
+        slot = next(slot);
+        const bool unit_end = c == geo.chunks - 1;
+        if (unit_end || j == n_steps - 1) {
+            // ---- end of this workgroup's piece of a unit: lane (g, b) of acc[nt][r]
+            // holds D[n0 + 32 wc + 16 nt + 4 g .. +3][b0 + 16 RT wr + 16 r + b]
+            const bool whole = piece_c0 == 0 && unit_end;
+            if (!whole) {
+                float *tile = part + (size_t)((int)blockIdx.x + unit) * T::kTile + (size_t)wave * (2 * RT * 256) + 4 * lane;
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)
+                        *(floatx4 *)(tile + (nt * RT + r) * 256) = acc[nt][r];
+            } else {
+                const int n0 = (unit % geo.n_blocks) * T::kCols + 32 * wc + 4 * g;
+                const int b0 = (unit / geo.n_blocks) * T::kRows + 16 * RT * wr + l16;
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)
+                        store4(out, acc[nt][r], b0 + 16 * r, n0 + 16 * nt, batch, N);
+            }
+            clear();
+            piece_c0 = 0;
+        }
+        if (unit_end) {
+            c = 0;
+            ++unit;
+        } else {
+            ++c;
+        }
+    }
+}
+
+// out of the units of out_proj_wide_kernel split between workgroups: the sum
+// of their pieces, workgroup by workgroup (one wave per 16 x 16 tile)
+template <typename E, int RT>
+__global__ __launch_bounds__(256) void reduce_wide_kernel(const float *__restrict__ part, E *__restrict__ out,
+                                                          int batch, int N, OutProjGeom geo)
+{
+    using T = Wide<RT>;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    const int t = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);  // (unit, wave, nt, r)
+    const int u = t / (16 * RT), ti = t - u * (16 * RT);
+    const int g_lo = u * geo.chunks / geo.per_wg, g_hi = (u * geo.chunks + geo.chunks - 1) / geo.per_wg;
+    if (g_lo == g_hi)  // one workgroup covered the unit and stored it
+        return;
+    const int wave = ti / (2 * RT), nt = ti / RT & 1, r = ti % RT;
+    const int b = (u / geo.n_blocks) * T::kRows + 16 * RT * (wave >> 2) + 16 * r + l16;
+    const int n = (u % geo.n_blocks) * T::kCols + 32 * (wave & 3) + 16 * nt + 4 * g;
+    const float *tile = part + (size_t)(g_lo + u) * T::kTile + (size_t)ti * 256 + 4 * lane;
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    // batches of 8 pieces whose loads are all in flight before the sums
+    for (int p0 = 0; p0 <= g_hi - g_lo; p0 += 8) {
+        floatx4 p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            p[i] = p0 + i <= g_hi - g_lo ? *(const floatx4 *)(tile + (size_t)(p0 + i) * T::kTile)
+                                         : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            v += p[i];
+    }
+    store4(out, v, b, n, batch, N);
+}
+
+OutProjGeom out_proj_geom(int n_blocks, int row_blocks, int chunks, int max_grid, int min_steps)
 {
     OutProjGeom geo;
-    geo.n_blocks = (N + kCols - 1) / kCols;
-    geo.chunks = (K + kChunk - 1) / kChunk;
-    geo.steps = geo.n_blocks * ((batch + 31) / 32) * geo.chunks;
-    const int grid = std::max(1, std::min({cu_count, kMaxGrid, geo.steps}));
-    geo.per_wg = (geo.steps + grid - 1) / grid;
+    geo.n_blocks = n_blocks;
+    geo.chunks = chunks;
+    geo.steps = n_blocks * row_blocks * chunks;
+    geo.per_wg = std::min(std::max((geo.steps + max_grid - 1) / max_grid, min_steps), geo.steps);
     geo.grid = (geo.steps + geo.per_wg - 1) / geo.per_wg;
     return geo;
+}
+
+// out_proj_kernel's units
+OutProjGeom narrow_geom(int batch, int K, int N, int max_grid)
+{
+    return out_proj_geom((N + kCols - 1) / kCols, (batch + 31) / 32, (K + kChunk - 1) / kChunk,
+                         std::min(max_grid, kMaxGrid), 1);
+}
+
+// out_proj_wide_kernel's, in equal row blocks of at most 256 rows
+constexpr int kWideMaxGrid = 256;  // the partial slots are sized for this many on any device
+// A workgroup's steps: with fewer a small W_O is cut so finely that the
+// partial tiles outweigh it, with more too few workgroups run (whole
+// projection, bf16, B = 160, n_h 16, d_model 2048, at 1 / 4 / 8 / 16:
+// 44.0 / 41.5 / 42.2 / 46.5 us; B = 33, n_h 16, d_model 1000: 18.0 / 12.9 /
+// 14.9 / 17.4).
+constexpr int kWideMinSteps = 4;
+
+// 32-row steps of a row block
+int wide_rt(int batch)
+{
+    const int blocks = (batch + 255) / 256;
+    return ((batch + blocks - 1) / blocks + 31) / 32;
+}
+
+OutProjGeom wide_geom(int batch, int K, int N, int max_grid)
+{
+    const int rows = 32 * wide_rt(batch);
+    return out_proj_geom((N + 127) / 128, (batch + rows - 1) / rows, K / 64, std::min(max_grid, kWideMaxGrid),
+                         kWideMinSteps);
+}
+
+// Whether a call takes the wide units. Up to 32 rows both forms stream W_O
+// once, and the narrow one's shorter prologue wins. Past that they win once
+// W_O holds kWideMinTotalSteps of their steps; below that W_O is at most
+// 8 MB and its re-reads hit the caches (whole projection, bf16, narrow -> wide: 256 steps, n_h 16, d_model
+// 1000: B = 33 11.6 -> 12.9 us, B = 64 16.9 -> 17.6, B = 256 58.2 -> 60.7;
+// 512 steps, n_h 16, d_model 2048, B = 160: 42.7 -> 41.5; 1024 steps, n_h 32,
+// d_model 2048, B = 40: 17.4 -> 16.5; n_h 128, d_model 5120: B = 40 69.4 ->
+// 49.7, B = 64 75.4 -> 55.4, B = 160 188.6 -> 96.0, B = 256 293 -> 135).
+constexpr int kWideMinTotalSteps = 512;
+
+bool use_wide(int batch, int K, int N)
+{
+    return batch > 32 && (int64_t)((N + 127) / 128) * (K / 64) >= kWideMinTotalSteps;
+}
+
+template <typename E, int RT>
+void launch_wide(const E *x, const E *w, E *out, float *part, int batch, int K, int N, hipStream_t s)
+{
+    const OutProjGeom geo = wide_geom(batch, K, N, current_cu_count());
+    hipLaunchKernelGGL((out_proj_wide_kernel<E, RT>), dim3(geo.grid), dim3(512), 0, s, x, w, out, part, batch, K, N, geo);
+    if (geo.per_wg % geo.chunks != 0 && geo.grid > 1)  // some unit is shared
+        hipLaunchKernelGGL((reduce_wide_kernel<E, RT>), dim3(geo.steps / geo.chunks * 4 * RT), dim3(256), 0, s, part, out,
+                           batch, N, geo);
+}
+
+template <typename E>
+void launch_out_proj(const E *x, const E *w, E *out, float *part, int batch, int K, int N, hipStream_t s)
+{
+    if (use_wide(batch, K, N)) {
+        switch (wide_rt(batch)) {
+        case 2: return launch_wide<E, 2>(x, w, out, part, batch, K, N, s);
+        case 3: return launch_wide<E, 3>(x, w, out, part, batch, K, N, s);
+        case 4: return launch_wide<E, 4>(x, w, out, part, batch, K, N, s);
+        case 5: return launch_wide<E, 5>(x, w, out, part, batch, K, N, s);
+        case 6: return launch_wide<E, 6>(x, w, out, part, batch, K, N, s);
+        case 7: return launch_wide<E, 7>(x, w, out, part, batch, K, N, s);
+        default: return launch_wide<E, 8>(x, w, out, part, batch, K, N, s);
+        }
+    }
+    const OutProjGeom geo = narrow_geom(batch, K, N, current_cu_count());
+    hipLaunchKernelGGL(out_proj_kernel<E>, dim3(geo.grid), dim3(256), 0, s, x, w, out, part, batch, K, N, geo);
+    const int quads = batch * ((N + 3) / 4);
+    if (geo.per_wg % geo.chunks != 0 && geo.grid > 1)
+        hipLaunchKernelGGL(reduce_units_kernel<E>, dim3((quads + 255) / 256), dim3(256), 0, s, part, out, batch, N, geo);
 }
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
@@ -439,6 +742,15 @@ int absorb(bool bf16, const void *q_nope, const void *q_rope, const void *w_uk, 
     return e == hipSuccess ? MLA_STATUS_SUCCESS : record_hip_error(e);
 }
 
+// o[b, h*128 + j] = O*[b, h, :] . W_UV[h][j][:], then out [B x d_model] = o W_O^T
+template <typename E>
+void project_typed(const E *o_star, const E *w_uv, const E *w_o, E *out, E *o, float *part, int batch, int num_heads,
+                   int d_model, hipStream_t s)
+{
+    hipLaunchKernelGGL(value_proj_kernel<E>, dim3(num_heads * 4), dim3(64), 0, s, o_star, w_uv, o, batch, num_heads);
+    launch_out_proj(o, w_o, out, part, batch, num_heads * kNope, d_model, s);
+}
+
 int project(bool bf16, const void *o_star, const void *w_uv, const void *w_o, void *out,
             void *workspace, size_t workspace_bytes, int batch, int num_heads, int d_model, void *stream)
 {
@@ -450,36 +762,17 @@ int project(bool bf16, const void *o_star, const void *w_uv, const void *w_o, vo
     if (workspace_bytes < mla_project_output_workspace_size(batch, num_heads, d_model))
         return MLA_STATUS_WORKSPACE_TOO_SMALL;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int hv = num_heads * kNope;
     // workspace: o [B x n_h*128] (16-bit), then the W_O kernel's partial tiles
-    const OutProjGeom geo = out_proj_geom(batch, hv, d_model, current_cu_count());
-    const bool split = geo.per_wg % geo.chunks != 0 && geo.grid > 1;  // some unit is shared
     char *ws = static_cast<char *>(workspace);
-    float *part = reinterpret_cast<float *>(ws + align256((size_t)batch * hv * 2));
-    const int quads = batch * ((d_model + 3) / 4);
-    // o[b, h*128 + j] = O*[b, h, :] . W_UV[h][j][:], then
-    // out [B x d_model] = o W_O^T
-    if (bf16) {
-        hipLaunchKernelGGL(value_proj_kernel<__bf16>, dim3(num_heads * 4), dim3(64), 0, s,
-                           static_cast<const __bf16 *>(o_star), static_cast<const __bf16 *>(w_uv),
-                           reinterpret_cast<__bf16 *>(ws), batch, num_heads);
-        hipLaunchKernelGGL(out_proj_kernel<__bf16>, dim3(geo.grid), dim3(256), 0, s,
-                           reinterpret_cast<const __bf16 *>(ws), static_cast<const __bf16 *>(w_o),
-                           static_cast<__bf16 *>(out), part, batch, hv, d_model, geo);
-        if (split)
-            hipLaunchKernelGGL(reduce_units_kernel<__bf16>, dim3((quads + 255) / 256), dim3(256), 0, s, part,
-                               static_cast<__bf16 *>(out), batch, d_model, geo);
-    } else {
-        hipLaunchKernelGGL(value_proj_kernel<_Float16>, dim3(num_heads * 4), dim3(64), 0, s,
-                           static_cast<const _Float16 *>(o_star), static_cast<const _Float16 *>(w_uv),
-                           reinterpret_cast<_Float16 *>(ws), batch, num_heads);
-        hipLaunchKernelGGL(out_proj_kernel<_Float16>, dim3(geo.grid), dim3(256), 0, s,
-                           reinterpret_cast<const _Float16 *>(ws), static_cast<const _Float16 *>(w_o),
-                           static_cast<_Float16 *>(out), part, batch, hv, d_model, geo);
-        if (split)
-            hipLaunchKernelGGL(reduce_units_kernel<_Float16>, dim3((quads + 255) / 256), dim3(256), 0, s, part,
-                               static_cast<_Float16 *>(out), batch, d_model, geo);
-    }
+    float *part = reinterpret_cast<float *>(ws + align256((size_t)batch * num_heads * kNope * 2));
+    if (bf16)
+        project_typed(static_cast<const __bf16 *>(o_star), static_cast<const __bf16 *>(w_uv),
+                      static_cast<const __bf16 *>(w_o), static_cast<__bf16 *>(out), reinterpret_cast<__bf16 *>(ws), part,
+                      batch, num_heads, d_model, s);
+    else
+        project_typed(static_cast<const _Float16 *>(o_star), static_cast<const _Float16 *>(w_uv),
+                      static_cast<const _Float16 *>(w_o), static_cast<_Float16 *>(out), reinterpret_cast<_Float16 *>(ws),
+                      part, batch, num_heads, d_model, s);
     const hipError_t e = hipPeekAtLastError();
     return e == hipSuccess ? MLA_STATUS_SUCCESS : record_hip_error(e);
 }
@@ -494,10 +787,17 @@ size_t mla_project_output_workspace_size(int batch, int num_heads, int d_model)
     if (batch < 1 || num_heads < 1 || num_heads > 4096 || d_model < 1)
         return 0;
     // the value projection [B x n_h*128] (16-bit), then the output
-    // projection's fp32 partial tiles (two per workgroup, at most kMaxGrid
-    // workgroups on any device)
-    const mla::OutProjGeom geo = mla::out_proj_geom(batch, num_heads * mla::kNope, d_model, mla::kMaxGrid);
-    return mla::align256((size_t)batch * num_heads * mla::kNope * 2) + (size_t)2 * geo.grid * mla::kPartTile * 4;
+    // projection's fp32 partial tiles: two per workgroup of at most kMaxGrid,
+    // or one per workgroup and unit, whatever the device
+    const int hv = num_heads * mla::kNope;
+    size_t part;
+    if (mla::use_wide(batch, hv, d_model)) {
+        const mla::OutProjGeom geo = mla::wide_geom(batch, hv, d_model, mla::kWideMaxGrid);
+        part = ((size_t)std::min(mla::kWideMaxGrid, geo.steps) + geo.steps / geo.chunks) * 128 * 32 * mla::wide_rt(batch) * 4;
+    } else {
+        part = (size_t)2 * mla::narrow_geom(batch, hv, d_model, mla::kMaxGrid).grid * mla::kPartTile * 4;
+    }
+    return mla::align256((size_t)batch * hv * 2) + part;
 }
 
 int mla_absorb_query_fp16(const void *q_nope, const void *q_rope, const void *w_uk, void *q_star, int batch,

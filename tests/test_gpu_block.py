@@ -60,6 +60,18 @@ def test_project_output(dtype, tol, b, n_h, d_model):
     np.testing.assert_allclose(got.double().cpu().numpy(), O.project_output(o_d, wuv_d, wo_d), atol=tol, rtol=tol)
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 1e-2), (torch.bfloat16, 3e-2)])
+# More than 32 rows: units of 128 columns x all rows. n_h = 16, d_model 2050:
+# units shared by workgroups, 2 columns in the last one (scalar stores), at the
+# first and the last row count of every height from 64 to 256, and two and
+# three row blocks; n_h = 2, d_model 32768 / 32767: every unit in one workgroup
+# (direct stores, vector and scalar); n_h = 1: two K chunks.
+@pytest.mark.parametrize("b,n_h,d_model", [(b, 16, 2050) for b in (33, 64, 65, 97, 128, 129, 161, 193, 225, 256, 257, 513)] +
+                         [(40, 2, 32768), (63, 2, 32767), (34, 1, 32768)])
+def test_project_output_wide(dtype, tol, b, n_h, d_model):
+    test_project_output(dtype, tol, b, n_h, d_model)
+
+
 @pytest.mark.parametrize("n_h", [16, 128])
 def test_decode_block_equals_unabsorbed_attention(n_h):
     # absorb -> batched decode -> project, against per-head attention with
