@@ -127,54 +127,77 @@ __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nop
     }
 }
 
-// Value up-projection, one wave per (head h, 32-row slice js of W_UV[h]):
+// Value up-projection:
 //   o[b, h * 128 + j] = sum_k O*[b, h, k] W_UV[h][j][k],
-// as its transpose D[j][b]: W_UV rows (k contiguous) are the A operand and
-// O* rows the B operand, both read from global memory; the 16 K-steps' A
-// operands and the B operands of the first 32 rows are loaded up front.
-template <typename E>
-__global__ __launch_bounds__(64) void value_proj_kernel(const E *__restrict__ o_star, const E *__restrict__ w_uv,
-                                                        E *__restrict__ o, int batch, int num_heads)
+// as its transpose D[j][b] on 16x16x32 MFMAs: W_UV rows (k contiguous) are the
+// A operand, 32 of them per wave, held in registers; O* rows the B operand.
+// One workgroup per (head, column group of NW waves, row group of up to TP
+// 16-row tiles). The rows (1 KB each) come into LDS by direct loads, 16-byte
+// chunk c of row r at c ^ (r mod 16), so that each crosses L2 once per column
+// group, and every load of the workgroup is in flight before the one wait for
+// them all: it is bound by the bytes and one memory round trip (B = 160, 128
+// heads, 43 MB: 46 -> 12 us against one-wave workgroups that loaded each
+// 16-row tile when they came to it; B = 32, 22 MB: 6.8 -> 5.9).
+template <typename E, int NW, int TP>
+__global__ __launch_bounds__(64 * NW) void value_proj_kernel(const E *__restrict__ o_star, const E *__restrict__ w_uv,
+                                                                E *__restrict__ o, int batch, int num_heads, int groups)
 {
     using E8 = typename Vec<E>::v8;
     using E4 = typename Vec<E>::v4;
-    const int h = blockIdx.x >> 2, js = blockIdx.x & 3;
-    const int lane = threadIdx.x, l16 = lane & 15, g = lane >> 4;
-    auto load_o = [&](int b, int kk) -> E8 {
-        return b < batch ? *(const E8 *)(o_star + ((size_t)b * num_heads + h) * kLatent + 32 * kk + 8 * g) : E8{};
-    };
-    // every load of the first two 16-row tiles is in flight at once
-    E8 a[2][kLatent / 32], o0[2][kLatent / 32];
+    constexpr int kSlices = 4 / NW;  // column groups per head
+    __shared__ __attribute__((aligned(1024))) E s_o[TP * 16 * kLatent];
+    // heads innermost, so that the workgroups of a head sit on one XCD (when n_h mod 8 = 0)
+    const int h = blockIdx.x % num_heads, rest = blockIdx.x / num_heads;
+    const int cs = rest % kSlices, rg = rest / kSlices;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j0 = 32 * (NW * cs + wave);
+    const int tiles = (batch + 15) / 16;
+    const int b0 = 16 * (rg * tiles / groups);
+    const int lim = min(16 * ((rg + 1) * tiles / groups), batch) - 1;  // this group's last row
+    E8 a[2][kLatent / 32];
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt) {
-        const E *wrow = w_uv + ((size_t)h * kNope + 32 * js + 16 * jt + l16) * kLatent + 8 * g;
+        const E *wrow = w_uv + ((size_t)h * kNope + j0 + 16 * jt + l16) * kLatent + 8 * g;
 #pragma unroll
         for (int kk = 0; kk < kLatent / 32; ++kk)
             a[jt][kk] = *(const E8 *)(wrow + 32 * kk);
     }
 #pragma unroll
-    for (int bt = 0; bt < 2; ++bt)
+    for (int i = 0; i < 16 * TP / NW; ++i) {
+        const int r = wave + NW * i;  // rows past the group's last re-read it and are not stored
+        global_to_lds16(o_star + ((size_t)min(b0 + r, lim) * num_heads + h) * kLatent, 16 * (lane ^ (r & 15)),
+                        s_o + r * kLatent);
+    }
+    MLA_WAIT_VMCNT(0);
+    lds_barrier();
+    floatx4 acc[2][TP];
 #pragma unroll
-        for (int kk = 0; kk < kLatent / 32; ++kk)
-            o0[bt][kk] = load_o(16 * bt + l16, kk);
-    for (int b0 = 0; b0 < batch; b0 += 16) {
-        const int b = b0 + l16;
-        floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+    for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-        for (int kk = 0; kk < kLatent / 32; ++kk) {
-            const E8 ov = b0 < 32 ? o0[b0 >> 4][kk] : load_o(b, kk);
+        for (int t = 0; t < TP; ++t)
+            acc[jt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < kLatent / 32; ++kk) {
+#pragma unroll
+        for (int t = 0; t < TP; ++t) {
+            const E8 ov = *(const E8 *)(s_o + (16 * t + l16) * kLatent + 8 * ((4 * kk + g) ^ l16));
 #pragma unroll
             for (int jt = 0; jt < 2; ++jt)
-                acc[jt] = mfma16x16x32(a[jt][kk], ov, acc[jt]);
+                acc[jt][t] = mfma16x16x32(a[jt][kk], ov, acc[jt][t]);
         }
-        // lane (g, b) holds D[j0 + 4 g .. +3][b]
-        if (b < batch) {
+    }
+    // lane (g, b) holds D[j0 + 16 jt + 4 g .. +3][b0 + 16 t + b]
 #pragma unroll
-            for (int jt = 0; jt < 2; ++jt) {
-                const int j = 32 * js + 16 * jt + 4 * g;
-                const E4 v = {(E)acc[jt][0], (E)acc[jt][1], (E)acc[jt][2], (E)acc[jt][3]};
-                *(E4 *)(o + (size_t)b * num_heads * kNope + (size_t)h * kNope + j) = v;
-            }
+    for (int t = 0; t < TP; ++t) {
+        const int b = b0 + 16 * t + l16;
+        if (b > lim)
+            continue;
+#pragma unroll
+        for (int jt = 0; jt < 2; ++jt) {
+            const floatx4 v = acc[jt][t];
+            *(E4 *)(o + (size_t)b * num_heads * kNope + (size_t)h * kNope + j0 + 16 * jt + 4 * g) =
+                E4{(E)v[0], (E)v[1], (E)v[2], (E)v[3]};
         }
     }
 }
@@ -742,12 +765,45 @@ int absorb(bool bf16, const void *q_nope, const void *q_rope, const void *w_uk, 
     return e == hipSuccess ? MLA_STATUS_SUCCESS : record_hip_error(e);
 }
 
+template <typename E, int NW>
+auto value_proj_for(int tp)
+{
+    switch (tp) {
+    case 1: return value_proj_kernel<E, NW, 1>;
+    case 2: return value_proj_kernel<E, NW, 2>;
+    case 3: return value_proj_kernel<E, NW, 3>;
+    case 4: return value_proj_kernel<E, NW, 4>;
+    case 5: return value_proj_kernel<E, NW, 5>;
+    case 6: return value_proj_kernel<E, NW, 6>;
+    case 7: return value_proj_kernel<E, NW, 7>;
+    default: return value_proj_kernel<E, NW, 8>;
+    }
+}
+
+// Row groups: as few as 8 tiles a workgroup allow, since each reads all of
+// W_UV again (at most 4 tiles, B = 160, 128 heads: 15.1 us against 12.3; 256:
+// 16.2 against 14.8), but 256 workgroups where the heads give fewer (n_h 16,
+// B = 256: 6.2 us with four groups, 10.6 with two; B = 32 3.6 with two, 4.1
+// with one). Then the widest column group that leaves 256 workgroups (two
+// column groups, 32 rows, 128 heads: 5.9 us against 6.4 with two row groups).
+template <typename E>
+void launch_value_proj(const E *o_star, const E *w_uv, E *o, int batch, int num_heads, hipStream_t s)
+{
+    const int tiles = (batch + 15) / 16;
+    const int groups = std::max((tiles + 7) / 8, std::min(tiles, (64 + num_heads - 1) / num_heads));
+    const int tp = (tiles + groups - 1) / groups;
+    const int nw = num_heads * groups >= 256 ? 4 : num_heads * groups >= 128 ? 2 : 1;
+    auto k = nw == 4 ? value_proj_for<E, 4>(tp) : nw == 2 ? value_proj_for<E, 2>(tp) : value_proj_for<E, 1>(tp);
+    hipLaunchKernelGGL(k, dim3(num_heads * (4 / nw) * groups), dim3(64 * nw), 0, s, o_star, w_uv, o, batch, num_heads,
+                       groups);
+}
+
 // o[b, h*128 + j] = O*[b, h, :] . W_UV[h][j][:], then out [B x d_model] = o W_O^T
 template <typename E>
 void project_typed(const E *o_star, const E *w_uv, const E *w_o, E *out, E *o, float *part, int batch, int num_heads,
                    int d_model, hipStream_t s)
 {
-    hipLaunchKernelGGL(value_proj_kernel<E>, dim3(num_heads * 4), dim3(64), 0, s, o_star, w_uv, o, batch, num_heads);
+    launch_value_proj(o_star, w_uv, o, batch, num_heads, s);
     launch_out_proj(o, w_o, out, part, batch, num_heads * kNope, d_model, s);
 }
 

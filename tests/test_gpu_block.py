@@ -61,6 +61,16 @@ def test_project_output(dtype, tol, b, n_h, d_model):
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float16, 1e-2), (torch.bfloat16, 3e-2)])
+# The value projection's row groups (up to 8 tiles of 16 rows, more groups when
+# there are few heads) and column groups (4, 2 or 1 waves of 32 columns): full
+# and ragged last tiles, uneven groups, head counts on both sides of each rule.
+@pytest.mark.parametrize("b,n_h", [(16, 1), (17, 5), (31, 40), (33, 63), (48, 64), (80, 65), (112, 100), (127, 127),
+                                   (128, 128), (129, 64), (144, 128), (200, 33), (272, 130), (16, 256), (100, 257)])
+def test_value_projection_groups(dtype, tol, b, n_h):
+    test_project_output(dtype, tol, b, n_h, 64)
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 1e-2), (torch.bfloat16, 3e-2)])
 # More than 32 rows: units of 128 columns x all rows. n_h = 16, d_model 2050:
 # units shared by workgroups, 2 columns in the last one (scalar stores), at the
 # first and the last row count of every height from 64 to 256, and two and
