@@ -655,13 +655,13 @@ __global__ __launch_bounds__(256) void reduce_wide_kernel(const float *__restric
     store4(out, v, b, n, batch, N);
 }
 
-OutProjGeom out_proj_geom(int n_blocks, int row_blocks, int chunks, int max_grid, int min_steps)
+OutProjGeom out_proj_geom(int n_blocks, int row_blocks, int chunks, int max_grid)
 {
     OutProjGeom geo;
     geo.n_blocks = n_blocks;
     geo.chunks = chunks;
     geo.steps = n_blocks * row_blocks * chunks;
-    geo.per_wg = std::min(std::max((geo.steps + max_grid - 1) / max_grid, min_steps), geo.steps);
+    geo.per_wg = (geo.steps + max_grid - 1) / max_grid;
     geo.grid = (geo.steps + geo.per_wg - 1) / geo.per_wg;
     return geo;
 }
@@ -670,18 +670,11 @@ OutProjGeom out_proj_geom(int n_blocks, int row_blocks, int chunks, int max_grid
 OutProjGeom narrow_geom(int batch, int K, int N, int max_grid)
 {
     return out_proj_geom((N + kCols - 1) / kCols, (batch + 31) / 32, (K + kChunk - 1) / kChunk,
-                         std::min(max_grid, kMaxGrid), 1);
+                         std::min(max_grid, kMaxGrid));
 }
 
 // out_proj_wide_kernel's, in equal row blocks of at most 256 rows
 constexpr int kWideMaxGrid = 256;  // the partial slots are sized for this many on any device
-// A workgroup's steps: with fewer a small W_O is cut so finely that the
-// partial tiles outweigh it, with more too few workgroups run (whole
-// projection, bf16, B = 160, n_h 16, d_model 2048, at 1 / 4 / 8 / 16:
-// 44.0 / 41.5 / 42.2 / 46.5 us; B = 33, n_h 16, d_model 1000: 18.0 / 12.9 /
-// 14.9 / 17.4).
-constexpr int kWideMinSteps = 4;
-
 // 32-row steps of a row block
 int wide_rt(int batch)
 {
@@ -692,19 +685,20 @@ int wide_rt(int batch)
 OutProjGeom wide_geom(int batch, int K, int N, int max_grid)
 {
     const int rows = 32 * wide_rt(batch);
-    return out_proj_geom((N + 127) / 128, (batch + rows - 1) / rows, K / 64, std::min(max_grid, kWideMaxGrid),
-                         kWideMinSteps);
+    return out_proj_geom((N + 127) / 128, (batch + rows - 1) / rows, K / 64, std::min(max_grid, kWideMaxGrid));
 }
 
 // Whether a call takes the wide units. Up to 32 rows both forms stream W_O
 // once, and the narrow one's shorter prologue wins. Past that they win once
-// W_O holds kWideMinTotalSteps of their steps; below that W_O is at most
-// 8 MB and its re-reads hit the caches (whole projection, bf16, narrow -> wide: 256 steps, n_h 16, d_model
-// 1000: B = 33 11.6 -> 12.9 us, B = 64 16.9 -> 17.6, B = 256 58.2 -> 60.7;
-// 512 steps, n_h 16, d_model 2048, B = 160: 42.7 -> 41.5; 1024 steps, n_h 32,
-// d_model 2048, B = 40: 17.4 -> 16.5; n_h 128, d_model 5120: B = 40 69.4 ->
-// 49.7, B = 64 75.4 -> 55.4, B = 160 188.6 -> 96.0, B = 256 293 -> 135).
-constexpr int kWideMinTotalSteps = 512;
+// W_O holds kWideMinTotalSteps of their steps (32 MB); below that its
+// re-reads hit the caches and the wide units' partial tiles weigh more (whole
+// projection, bf16, narrow / wide: 256 steps, n_h 16, d_model 1000: B = 64
+// 9.7 / 10.0 us, B = 256 16.7 / 18.6; 512 steps, d_model 2048: B = 64 11.1 /
+// 11.3, B = 256 19.1 / 23.3; 1024 steps, n_h 32: B = 40 13.8 / 15.4; 2048
+// steps, n_h 128, d_model 1000: B = 33 21.5 / 20.0, B = 64 22.6 / 21.6;
+// d_model 5120: B = 40 64.6 / 44.4, B = 64 66.1 / 46.1, B = 160 152 / 61.7,
+// B = 256 231 / 78.5).
+constexpr int kWideMinTotalSteps = 2048;
 
 bool use_wide(int batch, int K, int N)
 {

@@ -71,13 +71,13 @@ def test_value_projection_groups(dtype, tol, b, n_h):
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float16, 1e-2), (torch.bfloat16, 3e-2)])
-# More than 32 rows: units of 128 columns x all rows. n_h = 16, d_model 2050:
-# units shared by workgroups, 2 columns in the last one (scalar stores), at the
-# first and the last row count of every height from 64 to 256, and two and
-# three row blocks; n_h = 2, d_model 32768 / 32767: every unit in one workgroup
-# (direct stores, vector and scalar); n_h = 1: two K chunks.
-@pytest.mark.parametrize("b,n_h,d_model", [(b, 16, 2050) for b in (33, 64, 65, 97, 128, 129, 161, 193, 225, 256, 257, 513)] +
-                         [(40, 2, 32768), (63, 2, 32767), (34, 1, 32768)])
+# More than 32 rows and 32 MB of W_O: units of 128 columns x all rows. n_h = 16,
+# d_model 8194: units shared by workgroups, 2 columns in the last one (scalar
+# stores), at the first and the last row count of every height from 64 to 256,
+# and two and three row blocks; n_h = 2, d_model 65536 / 65535: every unit in
+# one workgroup (direct stores, vector and scalar); n_h = 1: two K chunks.
+@pytest.mark.parametrize("b,n_h,d_model", [(b, 16, 8194) for b in (33, 64, 65, 97, 128, 129, 161, 193, 225, 256, 257, 513)] +
+                         [(40, 2, 65536), (63, 2, 65535), (34, 1, 131072)])
 def test_project_output_wide(dtype, tol, b, n_h, d_model):
     test_project_output(dtype, tol, b, n_h, d_model)
 
