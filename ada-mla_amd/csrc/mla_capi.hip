@@ -56,13 +56,13 @@ int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // (16, 24, 32) 20.5 / 18.6 / 16.9; N = 4096 (24, 28, 32) 26.6 / 25.4 / 23.3.
 constexpr int kMinSplitTokensF32 = 32;
 
-// fp32 path: 32-head workgroups once their chunks hold this many tokens (12
-// blocks). Measured per call on one box (16 / 32 heads per workgroup, the
-// planner's split counts): n_h = 128, N = 4096 24.5 / 29.9 us, N = 8192
-// 36.0 / 38.1, N = 12288 45.6 / 45.4 (192-token chunks at 32 heads),
-// N = 16384 57.3 / 55.4; n_h = 64, N = 8192 23.9 / 27.6, N = 32768 57.4 /
-// 55.4; n_h = 32, N = 16384 22.3 / 26.0.
-constexpr int kHt32MinChunkTokensF32 = 192;
+// fp32 path: 32-head workgroups once their chunks hold this many tokens (8
+// blocks). Measured per call on one box (16 / 32 heads per workgroup, one
+// workgroup per CU): n_h = 128, N = 4096 (64-token chunks at 32 heads) 20.8 /
+// 23.7 us, N = 8192 (128) 29.4 / 27.7, N = 12288 (192) 36.6 / 30.8, N = 20011
+// 53.8 / 42.1; n_h = 64, N = 9290 (146) 22.2 / 22.7, N = 32768 44.8 / 36.3;
+// n_h = 32, N = 16384 (64) 19.2 / 20.7.
+constexpr int kHt32MinChunkTokensF32 = 128;
 
 constexpr size_t kAlign = 256;
 size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
