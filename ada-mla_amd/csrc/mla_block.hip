@@ -39,7 +39,8 @@ constexpr int kDK = kLatent + kRope;
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Absorption, one workgroup (4 waves) per (head h, 128-column slice cs):
+// Absorption, one workgroup (4 waves) per (head h, 128-column slice cs, row
+// group):
 //   Q*[b, h, 128 cs + n] = sum_k q_nope[b, h, k] W_UK[h][k][128 cs + n],
 // computed as its transpose D[n][b] on 16x16x32 MFMAs: the W_UK slice
 // (128 x 128) is staged in LDS, rows 256 bytes apart with 16-byte chunk c of
@@ -50,7 +51,7 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 template <typename E>
 __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nope, const E *__restrict__ q_rope,
                                                      const E *__restrict__ w_uk, E *__restrict__ q_star,
-                                                     int batch, int num_heads)
+                                                     int batch, int num_heads, int group_rows)
 {
     using E8 = typename Vec<E>::v8;
     using E4 = typename Vec<E>::v4;
@@ -58,17 +59,18 @@ __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nop
     const int h = blockIdx.x >> 2, cs = blockIdx.x & 3;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.y * group_rows, row1 = min(row0 + group_rows, batch);  // the group's rows
     // B operands of the first two 16-row tiles, requested before the weights
     // so that both round trips overlap: lane (g, b) holds q_nope[b0 + b][h][32 kk + 8 g .. +7]
     auto load_q = [&](int b, int kk) -> E8 {
-        return b < batch ? *(const E8 *)(q_nope + ((size_t)b * num_heads + h) * kNope + 32 * kk + 8 * g) : E8{};
+        return b < row1 ? *(const E8 *)(q_nope + ((size_t)b * num_heads + h) * kNope + 32 * kk + 8 * g) : E8{};
     };
     E8 q0[2][kNope / 32];
 #pragma unroll
     for (int bt = 0; bt < 2; ++bt)
 #pragma unroll
         for (int kk = 0; kk < kNope / 32; ++kk)
-            q0[bt][kk] = load_q(16 * bt + l16, kk);
+            q0[bt][kk] = load_q(row0 + 16 * bt + l16, kk);
     // stage W_UK[h][:, 128 cs .. +127]: 16-byte chunk c of row k (16 per row)
     const E *wsrc = w_uk + (size_t)h * kNope * kLatent + 128 * cs;
 #pragma unroll
@@ -77,8 +79,8 @@ __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nop
         *(uint4 *)(s_w + k * 128 + 8 * (c ^ (k & 15))) = *(const uint4 *)(wsrc + (size_t)k * kLatent + 8 * c);
     }
     if (cs == 0) {  // the rope columns, 8 chunks of 16 bytes per row
-        for (int i = tid; i < batch * 8; i += 256) {
-            const int b = i >> 3, c = i & 7;
+        for (int i = tid; i < (row1 - row0) * 8; i += 256) {
+            const int b = row0 + (i >> 3), c = i & 7;
             *(uint4 *)(q_star + ((size_t)b * num_heads + h) * kDK + kLatent + 8 * c) =
                 *(const uint4 *)(q_rope + ((size_t)b * num_heads + h) * kRope + 8 * c);
         }
@@ -102,13 +104,13 @@ __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nop
             a[nt][kk] = E8{part[0][0], part[0][1], part[0][2], part[0][3], part[1][0], part[1][1], part[1][2], part[1][3]};
         }
     }
-    for (int b0 = 0; b0 < batch; b0 += 16) {
-        const int b = b0 + l16;
+    for (int r = 0; r < row1 - row0; r += 16) {
+        const int b = row0 + r + l16;
         floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
         E8 qv[kNope / 32];
 #pragma unroll
         for (int kk = 0; kk < kNope / 32; ++kk)
-            qv[kk] = b0 < 32 ? q0[b0 >> 4][kk] : load_q(b, kk);
+            qv[kk] = r < 32 ? q0[r >> 4][kk] : load_q(b, kk);
 #pragma unroll
         for (int kk = 0; kk < kNope / 32; ++kk) {
 #pragma unroll
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nop
                 acc[nt] = mfma16x16x32(a[nt][kk], qv[kk], acc[nt]);
         }
         // lane (g, b) holds D[n0 + 4 g .. +3][b]
-        if (b < batch) {
+        if (b < row1) {
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt) {
                 const int n = 128 * cs + 32 * wave + 16 * nt + 4 * g;
@@ -738,6 +740,21 @@ void launch_out_proj(const E *x, const E *w, E *out, float *part, int batch, int
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
+// Row groups (multiples of 16 rows): so many that few heads still give 512
+// workgroups (n_h 16, B = 256: 14.0 us in one group, 5.8 in eight; n_h 32 15.4
+// and 9.3 in four). 128 heads keep one: each group stages W_UK again, and
+// requesting rows further ahead within one did not pay either (B = 256, two or
+// four tiles ahead: 25.9 and 27.7 us against 23.8).
+template <typename E>
+void launch_absorb(const E *q_nope, const E *q_rope, const E *w_uk, E *q_star, int batch, int num_heads, hipStream_t s)
+{
+    const int tiles = (batch + 15) / 16;
+    const int most = std::min(tiles, (128 + num_heads - 1) / num_heads);
+    const int rows = 16 * ((tiles + most - 1) / most);
+    hipLaunchKernelGGL(absorb_kernel<E>, dim3(num_heads * 4, (batch + rows - 1) / rows), dim3(256), 0, s, q_nope, q_rope,
+                       w_uk, q_star, batch, num_heads, rows);
+}
+
 int absorb(bool bf16, const void *q_nope, const void *q_rope, const void *w_uk, void *q_star,
            int batch, int num_heads, void *stream)
 {
@@ -748,13 +765,11 @@ int absorb(bool bf16, const void *q_nope, const void *q_rope, const void *w_uk, 
         return MLA_STATUS_MISALIGNED;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (bf16)
-        hipLaunchKernelGGL(absorb_kernel<__bf16>, dim3(num_heads * 4), dim3(256), 0, s,
-                           static_cast<const __bf16 *>(q_nope), static_cast<const __bf16 *>(q_rope),
-                           static_cast<const __bf16 *>(w_uk), static_cast<__bf16 *>(q_star), batch, num_heads);
+        launch_absorb(static_cast<const __bf16 *>(q_nope), static_cast<const __bf16 *>(q_rope),
+                      static_cast<const __bf16 *>(w_uk), static_cast<__bf16 *>(q_star), batch, num_heads, s);
     else
-        hipLaunchKernelGGL(absorb_kernel<_Float16>, dim3(num_heads * 4), dim3(256), 0, s,
-                           static_cast<const _Float16 *>(q_nope), static_cast<const _Float16 *>(q_rope),
-                           static_cast<const _Float16 *>(w_uk), static_cast<_Float16 *>(q_star), batch, num_heads);
+        launch_absorb(static_cast<const _Float16 *>(q_nope), static_cast<const _Float16 *>(q_rope),
+                      static_cast<const _Float16 *>(w_uk), static_cast<_Float16 *>(q_star), batch, num_heads, s);
     const hipError_t e = hipPeekAtLastError();
     return e == hipSuccess ? MLA_STATUS_SUCCESS : record_hip_error(e);
 }

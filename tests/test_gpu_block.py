@@ -42,6 +42,14 @@ def test_absorb_query(dtype, tol, b, n_h):
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float16, 1e-2), (torch.bfloat16, 3e-2)])
+# Row groups: none from 128 heads on, up to one per 16 rows with few; whole and
+# ragged last groups, three 16-row tiles and more in a group.
+@pytest.mark.parametrize("b,n_h", [(16, 127), (17, 127), (33, 64), (47, 5), (49, 43), (100, 1), (255, 16), (257, 16), (70, 130)])
+def test_absorb_query_row_groups(dtype, tol, b, n_h):
+    test_absorb_query(dtype, tol, b, n_h)
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float16, 1e-2), (torch.bfloat16, 3e-2)])
 # The W_O kernel cuts its (64-column unit, K-chunk) steps into equal ranges,
 # one per workgroup; on a 256-CU MI355X: (32, 128, 5120), the block workload,
 # splits units between 3-4 workgroups; (33, 16, 1000) one unit over 8 (two
