@@ -171,6 +171,18 @@ void splitkv_fp16_kernel(const E *__restrict__ q,
     // (Q* split, below); tiles of 16 heads convert C to fp16 for it instead,
     // where the split's fixed cost per piece exceeds what it saves
     constexpr bool kF8M = kF8 && HT >= 32;
+    // bf16, tiles of 32 or 64 heads: the two token halves' S waves keep one
+    // reference max between them (each takes the other's of the block before,
+    // and moves past it only by more than kLazyRescale), so that the O waves
+    // take P as stored in almost every block. In bf16 scaling P onto a reference
+    // costs them a conversion to fp32 and back per element (us per call, 128
+    // heads: 32 sequences of 512 .. 16384 tokens 86.8 -> 84.1, N = 131072 51.6
+    // -> 50.5; 64 heads, N = 20000, 32-head tiles 14.4 -> 14.2). 16-head tiles
+    // have that time to spare, and a short call pays for the exchange (N = 200
+    // 7.33 -> 7.47). In fp16 the scaling is one packed product, and the exchange
+    // gained nothing (batch 111.9 against 113.0, N = 131072 54.3 against 53.6,
+    // fp8 N = 65536 29.9 against 30.5).
+    constexpr bool kSharedRef = __is_same(E, __bf16) && HT >= 32;
     static_assert(kMode == kModeBatch || !kPaged, "a paged cache comes with cu_seqlens");
     static_assert(!(kF8 && (kPaged || !__is_same(E, _Float16))), "fp8 cache: packed layout, fp16 query");
     using E8 = typename Vec<E>::v8;
@@ -769,6 +781,14 @@ void splitkv_fp16_kernel(const E *__restrict__ q,
                     // ---- S^T tiles: tokens t0 + (0..15), heads of this wave.
                     // The 18 operand reads go out in batches of 3 K-steps,
                     // two batches ahead of the MFMAs that consume them.
+                    // kSharedRef: the other half's reference after the block before
+                    float m_other[T::kNS];
+                    if constexpr (kSharedRef) {
+#pragma unroll
+                        for (int ns = 0; ns < T::kNS; ++ns)
+                            m_other[ns] =
+                                blk > 0 ? s_m[(blk - 1) & 1][m_at(T::kSH * hg + 16 * ns + l16, 1 - th)] : -INFINITY;
+                    }
                     floatx4 acc[T::kNS][T::kChains];
 #pragma unroll
                     for (int ns = 0; ns < T::kNS; ++ns)
@@ -891,7 +911,13 @@ void splitkv_fp16_kernel(const E *__restrict__ q,
                             mx = fmaxf(mx, sv[i]);
                         }
                         mx = max_over_lane_groups(mx);
-                        const float mn = fmaxf(m_run[ns], mx);
+                        float mn;
+                        if constexpr (kSharedRef) {
+                            const float base = fmaxf(m_run[ns], m_other[ns]);
+                            mn = mx > base + kLazyRescale ? mx : base;
+                        } else {
+                            mn = fmaxf(m_run[ns], mx);
+                        }
                         // a half with no valid token yet keeps max -inf; its
                         // exponents are taken against 0 so that they are 0
                         const float ref = mn == -INFINITY ? 0.f : mn;
@@ -1182,37 +1208,61 @@ void splitkv_fp16_kernel(const E *__restrict__ q,
 #pragma unroll
                         for (int hs = 0; hs < T::kNHS; ++hs)
                             pb[hs] = *(const E8 *)(s_p[blk & 1] + (16 * hs + l16) * T::kPRow + 8 * g);
-                        // The reference only moves when a max passes it by more
-                        // than kLazyRescale (P scaled onto it then stays <= 2^8,
-                        // well inside fp16), so the rescale is rare.
-                        float alpha[T::kNHS];
-                        bool moved = false;
-#pragma unroll
-                        for (int hs = 0; hs < T::kNHS; ++hs) {
-                            const float mn = fmaxf(m0[hs], m1[hs]);  // finite: token p_lo is in half 0
-                            const bool up = mn > m_ref[hs] + kLazyRescale;  // always at the first block
-                            alpha[hs] = up ? fast_exp2(m_ref[hs] - mn) : 1.0f;
-                            moved |= up;
-                            if (up)
-                                m_ref[hs] = mn;
-                            const float f = fast_exp2((g < 2 ? m0[hs] : m1[hs]) - m_ref[hs]);
+                        auto scale_p = [](E8 &p, float f) {
                             if constexpr (__is_same(E, _Float16)) {
-                                pb[hs] *= (E)f;
+                                p *= (E)f;
                             } else {
                                 // bf16: scale in fp32, so that the factor is not
                                 // itself rounded to 8 bits (one error for the
                                 // whole half-block)
 #pragma unroll
                                 for (int i = 0; i < 8; ++i)
-                                    pb[hs][i] = (E)((float)pb[hs][i] * f);
+                                    p[i] = (E)((float)p[i] * f);
                             }
-                        }
-                        if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+                        };
+                        if constexpr (kSharedRef) {
+                            // P is taken as it is while both halves stand at the
+                            // accumulator's reference, which follows theirs
+                            bool moved = false;
 #pragma unroll
                             for (int hs = 0; hs < T::kNHS; ++hs)
+                                moved |= m0[hs] != m_ref[hs] || m1[hs] != m_ref[hs];
+                            if (__builtin_amdgcn_ballot_w64(moved) != 0) {
 #pragma unroll
-                                for (int dt = 0; dt < 8; ++dt)
-                                    o[hs][dt] *= alpha[hs];
+                                for (int hs = 0; hs < T::kNHS; ++hs) {
+                                    const float mn = fmaxf(m_ref[hs], fmaxf(m0[hs], m1[hs]));  // finite: token p_lo is in half 0
+                                    const float alpha = mn == m_ref[hs] ? 1.0f : fast_exp2(m_ref[hs] - mn);
+                                    m_ref[hs] = mn;
+                                    const float f = fast_exp2((g < 2 ? m0[hs] : m1[hs]) - mn);
+                                    scale_p(pb[hs], f);
+#pragma unroll
+                                    for (int dt = 0; dt < 8; ++dt)
+                                        o[hs][dt] *= alpha;
+                                }
+                            }
+                        } else {
+                            // The reference only moves when a max passes it by more
+                            // than kLazyRescale (P scaled onto it then stays <= 2^8,
+                            // well inside fp16), so the rescale is rare.
+                            float alpha[T::kNHS];
+                            bool moved = false;
+#pragma unroll
+                            for (int hs = 0; hs < T::kNHS; ++hs) {
+                                const float mn = fmaxf(m0[hs], m1[hs]);  // finite: token p_lo is in half 0
+                                const bool up = mn > m_ref[hs] + kLazyRescale;  // always at the first block
+                                alpha[hs] = up ? fast_exp2(m_ref[hs] - mn) : 1.0f;
+                                moved |= up;
+                                if (up)
+                                    m_ref[hs] = mn;
+                                scale_p(pb[hs], fast_exp2((g < 2 ? m0[hs] : m1[hs]) - m_ref[hs]));
+                            }
+                            if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+#pragma unroll
+                                for (int hs = 0; hs < T::kNHS; ++hs)
+#pragma unroll
+                                    for (int dt = 0; dt < 8; ++dt)
+                                        o[hs][dt] *= alpha[hs];
+                            }
                         }
                         // the page of the block the next step issues: read after
                         // this step's P and max reads (a scalar load shares the

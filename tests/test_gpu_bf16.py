@@ -152,3 +152,25 @@ def test_bf16_extension_dispatch():
     one = capi.decode_split_bf16(q.contiguous(), c[700:].contiguous())
     torch.cuda.synchronize()
     assert (got[1].float() - one.float()).abs().max().item() < 2e-2
+
+
+def _profile(name, n):
+    t = np.arange(n)
+    return {"up": 12.0 * (t // 32 % 6), "down": -12.0 * (t // 32 % 6), "halves": 16.0 * (t // 16 % 2),
+            "spike": np.where(t % 160 == 97, 60.0, 0.0), "two_spikes": np.where(t % 160 == 70, 40.0, 0.0) + np.where(t % 160 == 90, 70.0, 0.0),
+            "slope": 0.25 * (t % 320)}[name]
+
+
+# The reference max that the two token halves keep between them: logits that move
+# it in the first block, in every block, in one half only, in both halves of a
+# block, down, and slowly within its slack; at 64- and 32-head tiles.
+@pytest.mark.parametrize("n_h,n,splits,tile", [(128, 20480, 128, 64), (64, 20000, 0, 32)])
+@pytest.mark.parametrize("name", ["up", "down", "halves", "spike", "two_spikes", "slope"])
+def test_bf16_moving_reference(n_h, n, splits, tile, name):
+    print(f"bf16 {name} n_h={n_h}", flush=True)
+    assert capi.load().mla_decode_split_head_tile(n_h, n, splits, 0) == tile
+    q, c, _, _ = _bf16_inputs(n_h, n, seed=77)
+    # column 575 (rope: no output) adds the profile to every logit, in log2 units
+    q[:, 575] = 16.0
+    c[:, 575] = torch.from_numpy(_profile(name, n) * (192 ** 0.5 / 16.0 / 1.4426950408889634)).to(torch.bfloat16).cuda()
+    _check(_run(q, c, num_splits=splits), O.closed_form(q.double().cpu().numpy(), c.double().cpu().numpy()), name)
