@@ -141,6 +141,16 @@ constexpr double kDirectFixedUs = 7.0;
 // 108 -> 139 splits 71.3 -> 58.5 us; n_h = 32, N = 65536 114 -> 128 splits
 // 23.1 -> 20.8 us, N = 262144 (16, 108) -> (32, 179) 71.2 -> 59.0 us.
 constexpr double kStreamBytesPerUs = 7.5e6;  // n_h = 16 streams C at 7.7 TB/s in the steady state
+// Calls with cu_seqlens, fitted over 184 mixes of 2 .. 128 sequences of 0 ..
+// 16384 tokens at 16 .. 128 heads: against 0.25e-6 and 0, the charge of a
+// single sequence, the calls ran x0.988 by geomean. The plans it moves hold
+// short sequences: they go from 64-head tiles x 120 .. 128 chunks, which cut
+// most sequences in two, to 32-head tiles x 64 (128 heads: 64 sequences of 1 ..
+// 1500 tokens 35.9 -> 32.7 us, 17 of 2215 28.7 -> 24.9, 98 of 205 30.7 -> 27.8;
+// 64 heads, 86 of 841 32.2 -> 28.7; the worst, 64 heads, 17 of 335, 12.4 ->
+// 12.8). 0.35e-6 and 3 gave x0.991, 0.6e-6 and 3 x0.986 but 6% losses.
+constexpr double kBatchPartialUsPerByte = 0.4e-6;
+constexpr double kBatchPiecesUs64 = 4.0;
 double modelled_us(const Plan &p, int num_heads, int total_tokens, int batch, int cu_count, bool paged,
                    bool direct_ok, int c_bytes)
 {
@@ -165,7 +175,12 @@ double modelled_us(const Plan &p, int num_heads, int total_tokens, int batch, in
     const double chunks_live = std::min((double)wgs, (double)cu_count) / p.n_head_tiles;
     const double block_us = std::max(step_us * share, chunks_live * p.block_tokens * kDK * c_bytes / kStreamBytesPerUs);
     const double loop_us = rounds * steps * block_us;
-    return 11.0 + loop_us + 0.25e-6 * partial_bytes + 1.0 * combine_trips;
+    // a batch: its partials cost more per byte (its combine is bound by them),
+    // and the pieces of a 64-head chunk more than their virtual tokens
+    const bool seqlens = p.seq_cost > 0;
+    const double us_per_byte = seqlens ? kBatchPartialUsPerByte : 0.25e-6;
+    const double pieces_us = seqlens && p.head_tile == 64 ? kBatchPiecesUs64 * batch / p.n_chunks : 0.0;
+    return 11.0 + loop_us + us_per_byte * partial_bytes + 1.0 * combine_trips + pieces_us;
 }
 
 }  // namespace
