@@ -42,12 +42,19 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // Absorption, one workgroup (4 waves) per (head h, 128-column slice cs, row
 // group):
 //   Q*[b, h, 128 cs + n] = sum_k q_nope[b, h, k] W_UK[h][k][128 cs + n],
-// computed as its transpose D[n][b] on 16x16x32 MFMAs: the W_UK slice
-// (128 x 128) is staged in LDS, rows 256 bytes apart with 16-byte chunk c of
-// row k at c ^ (k mod 16), and read as the A operand (n x k) with the LDS
-// transpose read; q_nope rows are the B operand, read from global memory.
-// Wave w owns columns 32 w .. +31 (two 16-column tiles) for all B rows.
+// computed as its transpose D[n][b] on 16x16x32 MFMAs. The W_UK slice (128 x
+// 128) and the q_nope rows, kAbsorbTiles tiles of 16 at a time, come into LDS by
+// direct loads that are all in flight before one wait: rows are 256 bytes, with
+// 16-byte chunk c of row r at c ^ (r mod 16). W_UK is read as the A operand (n
+// x k) with the LDS transpose read, q_nope as the B operand.
+// Wave w owns columns 32 w .. +31 (two 16-column tiles) for all rows. It is
+// bound by the bytes (16.8 MB of W_UK and 196 KB a row at 128 heads) and one
+// memory round trip: against rows loaded by every wave for itself and 8-byte
+// stores, B = 32, 128 heads 6.3 -> 5.9 us, B = 256 23.9 -> 16.4 (the 16-byte
+// stores 2.5 us of it).
 // The slice cs = 0 also copies the 64 rope columns of each row.
+constexpr int kAbsorbTiles = 4;
+
 template <typename E>
 __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nope, const E *__restrict__ q_rope,
                                                      const E *__restrict__ w_uk, E *__restrict__ q_star,
@@ -55,29 +62,30 @@ __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nop
 {
     using E8 = typename Vec<E>::v8;
     using E4 = typename Vec<E>::v4;
-    __shared__ __attribute__((aligned(16))) E s_w[kNope * 128];
+    __shared__ __attribute__((aligned(1024))) E s_w[kNope * 128];
+    __shared__ __attribute__((aligned(1024))) E s_q[kAbsorbTiles * 16 * kNope];
     const int h = blockIdx.x >> 2, cs = blockIdx.x & 3;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, g = lane >> 4;
     const int row0 = blockIdx.y * group_rows, row1 = min(row0 + group_rows, batch);  // the group's rows
-    // B operands of the first two 16-row tiles, requested before the weights
-    // so that both round trips overlap: lane (g, b) holds q_nope[b0 + b][h][32 kk + 8 g .. +7]
-    auto load_q = [&](int b, int kk) -> E8 {
-        return b < row1 ? *(const E8 *)(q_nope + ((size_t)b * num_heads + h) * kNope + 32 * kk + 8 * g) : E8{};
+    // load units of 4 rows: lane -> row lane / 16, stored chunk lane mod 16
+    auto load_tiles = [&](int r) {
+        const E *base = q_nope + ((size_t)row0 * num_heads + h) * kNope;
+        const int ru = 4 * wave + g;  // row within a tile (rows past the group re-read its last one)
+#pragma unroll
+        for (int t = 0; t < kAbsorbTiles; ++t)
+            if (r + 16 * t < row1 - row0)
+                global_to_lds16(base, min(r + 16 * t + ru, row1 - 1 - row0) * num_heads * (kNope * 2) + 16 * (l16 ^ ru),
+                                s_q + (16 * t + 4 * wave) * kNope);
     };
-    E8 q0[2][kNope / 32];
-#pragma unroll
-    for (int bt = 0; bt < 2; ++bt)
-#pragma unroll
-        for (int kk = 0; kk < kNope / 32; ++kk)
-            q0[bt][kk] = load_q(row0 + 16 * bt + l16, kk);
-    // stage W_UK[h][:, 128 cs .. +127]: 16-byte chunk c of row k (16 per row)
     const E *wsrc = w_uk + (size_t)h * kNope * kLatent + 128 * cs;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int lin = tid + 256 * i, k = lin >> 4, c = lin & 15;
-        *(uint4 *)(s_w + k * 128 + 8 * (c ^ (k & 15))) = *(const uint4 *)(wsrc + (size_t)k * kLatent + 8 * c);
+        const int k = 32 * wave + 4 * i + g;
+        global_to_lds16(wsrc, k * (kLatent * 2) + 16 * (l16 ^ (k & 15)), s_w + (32 * wave + 4 * i) * 128);
     }
+    load_tiles(0);
     if (cs == 0) {  // the rope columns, 8 chunks of 16 bytes per row
         for (int i = tid; i < (row1 - row0) * 8; i += 256) {
             const int b = row0 + (i >> 3), c = i & 7;
@@ -85,45 +93,49 @@ __global__ __launch_bounds__(256) void absorb_kernel(const E *__restrict__ q_nop
                 *(const uint4 *)(q_rope + ((size_t)b * num_heads + h) * kRope + 8 * c);
         }
     }
-    __syncthreads();
-    // A operands (n x k): lane (g, i) holds W[32 kk + 8 g .. +7][n0 + i], from
-    // two transpose reads of 4 rows each
+    MLA_WAIT_VMCNT(0);
+    lds_barrier();
+    // A operands (n x k): row i of tile nt is column 8 (i / 4) + 4 nt + i mod 4
+    // of the wave's 32, so that a lane ends up with 8 adjacent columns; lane
+    // (g, i) holds W[32 kk + 8 g .. +7] of it, from two transpose reads of 4 rows
     E8 a[2][kNope / 32];
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
-        const int n0 = 32 * wave + 16 * nt;
 #pragma unroll
         for (int kk = 0; kk < kNope / 32; ++kk) {
             E4 part[2];
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf) {
                 const int row = 32 * kk + 8 * g + 4 * hf + (l16 >> 2);
-                const int col = n0 + 4 * (l16 & 3);  // 4 columns, 8 bytes
+                const int col = 32 * wave + 8 * (l16 & 3) + 4 * nt;  // 4 columns, 8 bytes
                 part[hf] = lds_read_tr16<E>(s_w + row * 128 + 8 * ((col >> 3) ^ (row & 15)) + (col & 7));
             }
             a[nt][kk] = E8{part[0][0], part[0][1], part[0][2], part[0][3], part[1][0], part[1][1], part[1][2], part[1][3]};
         }
     }
-    for (int r = 0; r < row1 - row0; r += 16) {
-        const int b = row0 + r + l16;
-        floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
-        E8 qv[kNope / 32];
-#pragma unroll
-        for (int kk = 0; kk < kNope / 32; ++kk)
-            qv[kk] = r < 32 ? q0[r >> 4][kk] : load_q(b, kk);
-#pragma unroll
-        for (int kk = 0; kk < kNope / 32; ++kk) {
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-                acc[nt] = mfma16x16x32(a[nt][kk], qv[kk], acc[nt]);
+    for (int r = 0; r < row1 - row0; r += 16 * kAbsorbTiles) {
+        if (r > 0) {
+            lds_barrier();  // every wave has read the tiles before
+            load_tiles(r);
+            MLA_WAIT_VMCNT(0);
+            lds_barrier();
         }
-        // lane (g, b) holds D[n0 + 4 g .. +3][b]
-        if (b < row1) {
+        const int tiles = min((row1 - row0 - r + 15) / 16, kAbsorbTiles);
+        for (int t = 0; t < tiles; ++t) {
+            floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                const int n = 128 * cs + 32 * wave + 16 * nt + 4 * g;
-                const E4 v = {(E)acc[nt][0], (E)acc[nt][1], (E)acc[nt][2], (E)acc[nt][3]};
-                *(E4 *)(q_star + ((size_t)b * num_heads + h) * kDK + n) = v;
+            for (int kk = 0; kk < kNope / 32; ++kk) {
+                const E8 qv = *(const E8 *)(s_q + (16 * t + l16) * kNope + 8 * ((4 * kk + g) ^ l16));
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt)
+                    acc[nt] = mfma16x16x32(a[nt][kk], qv, acc[nt]);
+            }
+            // lane (g, b) holds columns 8 g + 4 nt .. +3 of row b
+            const int b = row0 + r + 16 * t + l16;
+            if (b < row1) {
+                const E8 v = {(E)acc[0][0], (E)acc[0][1], (E)acc[0][2], (E)acc[0][3],
+                              (E)acc[1][0], (E)acc[1][1], (E)acc[1][2], (E)acc[1][3]};
+                *(E8 *)(q_star + ((size_t)b * num_heads + h) * kDK + 128 * cs + 32 * wave + 8 * g) = v;
             }
         }
     }
@@ -145,7 +157,6 @@ __global__ __launch_bounds__(64 * NW) void value_proj_kernel(const E *__restrict
                                                                 E *__restrict__ o, int batch, int num_heads, int groups)
 {
     using E8 = typename Vec<E>::v8;
-    using E4 = typename Vec<E>::v4;
     constexpr int kSlices = 4 / NW;  // column groups per head
     __shared__ __attribute__((aligned(1024))) E s_o[TP * 16 * kLatent];
     // heads innermost, so that the workgroups of a head sit on one XCD (when n_h mod 8 = 0)
@@ -157,19 +168,21 @@ __global__ __launch_bounds__(64 * NW) void value_proj_kernel(const E *__restrict
     const int tiles = (batch + 15) / 16;
     const int b0 = 16 * (rg * tiles / groups);
     const int lim = min(16 * ((rg + 1) * tiles / groups), batch) - 1;  // this group's last row
+    // row i of A tile jt is column 8 (i / 4) + 4 jt + i mod 4 of the wave's 32,
+    // so that a lane ends up with 8 adjacent columns
     E8 a[2][kLatent / 32];
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt) {
-        const E *wrow = w_uv + ((size_t)h * kNope + j0 + 16 * jt + l16) * kLatent + 8 * g;
+        const E *wrow = w_uv + ((size_t)h * kNope + j0 + 8 * (l16 >> 2) + 4 * jt + (l16 & 3)) * kLatent + 8 * g;
 #pragma unroll
         for (int kk = 0; kk < kLatent / 32; ++kk)
             a[jt][kk] = *(const E8 *)(wrow + 32 * kk);
     }
 #pragma unroll
     for (int i = 0; i < 16 * TP / NW; ++i) {
-        const int r = wave + NW * i;  // rows past the group's last re-read it and are not stored
-        global_to_lds16(o_star + ((size_t)min(b0 + r, lim) * num_heads + h) * kLatent, 16 * (lane ^ (r & 15)),
-                        s_o + r * kLatent);
+        const int r = wave + NW * i;  // rows past the group's last stay as they are: theirs is not stored
+        if (b0 + r <= lim)
+            global_to_lds16(o_star + ((size_t)(b0 + r) * num_heads + h) * kLatent, 16 * (lane ^ (r & 15)), s_o + r * kLatent);
     }
     MLA_WAIT_VMCNT(0);
     lds_barrier();
@@ -189,18 +202,15 @@ __global__ __launch_bounds__(64 * NW) void value_proj_kernel(const E *__restrict
                 acc[jt][t] = mfma16x16x32(a[jt][kk], ov, acc[jt][t]);
         }
     }
-    // lane (g, b) holds D[j0 + 16 jt + 4 g .. +3][b0 + 16 t + b]
+    // lane (g, b) holds columns j0 + 8 g + 4 jt .. +3 of row b0 + 16 t + b
 #pragma unroll
     for (int t = 0; t < TP; ++t) {
         const int b = b0 + 16 * t + l16;
         if (b > lim)
             continue;
-#pragma unroll
-        for (int jt = 0; jt < 2; ++jt) {
-            const floatx4 v = acc[jt][t];
-            *(E4 *)(o + (size_t)b * num_heads * kNope + (size_t)h * kNope + j0 + 16 * jt + 4 * g) =
-                E4{(E)v[0], (E)v[1], (E)v[2], (E)v[3]};
-        }
+        const floatx4 v = acc[0][t], u = acc[1][t];
+        *(E8 *)(o + (size_t)b * num_heads * kNope + (size_t)h * kNope + j0 + 8 * g) =
+            E8{(E)v[0], (E)v[1], (E)v[2], (E)v[3], (E)u[0], (E)u[1], (E)u[2], (E)u[3]};
     }
 }
 
@@ -741,10 +751,10 @@ void launch_out_proj(const E *x, const E *w, E *out, float *part, int batch, int
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Row groups (multiples of 16 rows): so many that few heads still give 512
-// workgroups (n_h 16, B = 256: 14.0 us in one group, 5.8 in eight; n_h 32 15.4
-// and 9.3 in four). 128 heads keep one: each group stages W_UK again, and
-// requesting rows further ahead within one did not pay either (B = 256, two or
-// four tiles ahead: 25.9 and 27.7 us against 23.8).
+// workgroups (n_h 16, B = 256: 13.8 us in one group with rows loaded per wave,
+// 4.3 in eight; n_h 32 15.4 and 6.4 in four). 128 heads keep one, as each group
+// brings W_UK into LDS again (B = 256, four groups of four tiles: 27.8 us
+// against 23.9 in one, both with rows loaded per wave).
 template <typename E>
 void launch_absorb(const E *q_nope, const E *q_rope, const E *w_uk, E *q_star, int batch, int num_heads, hipStream_t s)
 {
