@@ -140,6 +140,7 @@ constexpr double kDirectFixedUs = 7.0;
 // box: n_h = 16, N = 65536 114 -> 137 splits 22.9 -> 20.3 us, N = 262144
 // 108 -> 139 splits 71.3 -> 58.5 us; n_h = 32, N = 65536 114 -> 128 splits
 // 23.1 -> 20.8 us, N = 262144 (16, 108) -> (32, 179) 71.2 -> 59.0 us.
+constexpr int kXcds = 8;
 constexpr double kStreamBytesPerUs = 7.5e6;  // n_h = 16 streams C at 7.7 TB/s in the steady state
 // Calls with cu_seqlens, fitted over 184 mixes of 2 .. 128 sequences of 0 ..
 // 16384 tokens at 16 .. 128 heads: against 0.25e-6 and 0, the charge of a
@@ -160,7 +161,10 @@ double modelled_us(const Plan &p, int num_heads, int total_tokens, int batch, in
                                     (p.head_tile == 64 ? 1.5 : p.head_tile == 32 ? 0.88 : 0.65);
     const double step_us = p.head_tile == 64 ? 1.5 : p.head_tile == 32 ? 0.88 : 0.65;
     const int wgs = p.n_chunks * p.n_head_tiles;
-    const double rounds = std::ceil((double)wgs / cu_count);
+    // the tiles of a chunk share an XCD, so the XCDs with one chunk more decide
+    const double rounds = p.xcd_remap && cu_count % kXcds == 0
+                              ? std::ceil((double)ceil_div(p.n_chunks, kXcds) * p.n_head_tiles / (cu_count / kXcds))
+                              : std::ceil((double)wgs / cu_count);
     const double steps = std::ceil((double)p.chunk / p.block_tokens) + (paged ? 2.0 : 1.0);
     const double share = (p.n_head_tiles > 1 && !p.xcd_remap) ? 1.3 : 1.0;
     const double partial_bytes = (double)p.n_slots * num_heads * (kDV * p.part_bytes + 8);
@@ -187,6 +191,18 @@ double modelled_us(const Plan &p, int num_heads, int total_tokens, int batch, in
 
 namespace {
 
+// The most chunks of n_head_tiles workgroups that run in one round, the tiles of
+// a chunk on one XCD: with 3 tiles (48 heads by 16, 192 by 64) 10 chunks on the 32
+// CUs of an XCD, 80 in all. 85 (256 / 3) put 11 on five XCDs, whose 33rd
+// workgroup was a second round (us per call, 85 / 80
+// chunks: fp16, 48 heads, N = 57593 31.8 / 19.6, 192 heads, N = 21664 34.6 /
+// 20.5; 5 tiles, 51 / 48: 80 heads, N = 65080 48.7 / 29.5).
+int most_chunks(int cu_count, int n_head_tiles)
+{
+    const int per_xcd = cu_count % kXcds == 0 ? cu_count / kXcds / n_head_tiles : 0;
+    return std::max(1, per_xcd > 0 ? kXcds * per_xcd : cu_count / n_head_tiles);
+}
+
 Plan compute_plan(bool fp32, int num_heads, int total_tokens, int batch, bool seqlens,
                   int num_splits, int cu_count, CacheKind cache, bool f32_partials)
 {
@@ -211,7 +227,7 @@ Plan compute_plan(bool fp32, int num_heads, int total_tokens, int batch, bool se
         auto splits_for = [&](int ht) {
             if (num_splits > 0)
                 return num_splits;
-            const int per_round = std::max(1, cu_count / (num_heads / ht));
+            const int per_round = most_chunks(cu_count, num_heads / ht);
             return std::min(per_round, ceil_div(total_tokens, kMinSplitTokensF32));
         };
         // 32 heads per workgroup fill each C block once for twice the heads,
@@ -286,7 +302,7 @@ Plan compute_plan(bool fp32, int num_heads, int total_tokens, int batch, bool se
         const double step_us = p16.head_tile == 64 ? 1.5 : p16.head_tile == 32 ? 0.88 : 0.65;
         const double live = std::min((double)p16.n_chunks * p16.n_head_tiles, (double)cu_count) / p16.n_head_tiles;
         if (live * p16.block_tokens * kDK * 2 / kStreamBytesPerUs > step_us)
-            set_chunks(p16, total_tokens + p16.seq_cost * batch, batch, std::max(1, cu_count / p16.n_head_tiles));
+            set_chunks(p16, total_tokens + p16.seq_cost * batch, batch, most_chunks(cu_count, p16.n_head_tiles));
     }
     if (cache != CacheKind::kF8 || num_splits > 0)
         return p16;

@@ -412,3 +412,18 @@ def test_fp8_workspace_size_covers_the_single_sequence_entry(n):
                                               None)
         assert st == capi.STATUS_HIP_ERROR, (n, flagless_splits, st)
     assert ws > 0
+
+
+@pytest.mark.parametrize("n_h", [16, 48, 80, 96, 128, 160, 192, 240, 256])
+def test_one_round_plans_fit_every_xcd(n_h):
+    """A single sequence's plan that leaves CUs over runs in one round on every
+    XCD: the head tiles of a chunk share one of 8 XCDs of 32 CUs, and chunks go
+    to the XCDs in turn, so ceil(chunks / 8) x tiles workgroups is the most that
+    an XCD gets."""
+    lib = capi.load()
+    for flags in (0, capi.FLAG_FP32_PARTIALS, capi.FLAG_FP8_CACHE):
+        for n in (1, 511, 2048, 8191, 21664, 57593, 131072):
+            chunks = lib.mla_decode_split_num_splits(n_h, n, 0, flags)
+            tiles = n_h // lib.mla_decode_split_head_tile(n_h, n, 0, flags)
+            if chunks * tiles <= 256:
+                assert -(-chunks // 8) * tiles <= 32, (flags, n, chunks, tiles)
