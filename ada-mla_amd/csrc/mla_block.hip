@@ -14,12 +14,12 @@
 //
 // These are weight-streaming GEMMs with M = B rows, all MFMA kernels of this
 // file: the two per-head ones (W_UK, W_UV: 128 KB of weights per head) one
-// workgroup per (head, column slice), with the rope columns of Q* copied by
-// the absorption kernel; the output projection (one [B x n_h*128] x
-// [n_h*128 x d_model] product, W_O streamed once from HBM) 32 output
-// columns per workgroup. fp16 / bf16 inputs, fp32 accumulation. No
-// reference code exists for this part (the reference stops at the decode
-// kernel).
+// workgroup per (head, column slice, row group), with the rope columns of Q*
+// copied by the absorption kernel; the output projection (one [B x n_h*128] x
+// [n_h*128 x d_model] product, bound by streaming W_O) stream-K over units of
+// 64 columns x 32 rows, or 128 columns x up to 256 rows. fp16 / bf16
+// inputs, fp32 accumulation. No reference code exists for this part (the
+// reference stops at the decode kernel).
 #include <algorithm>
 #include <cstdint>
 #include <type_traits>
@@ -166,8 +166,11 @@ __global__ __launch_bounds__(64 * NW) void value_proj_kernel(const E *__restrict
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j0 = 32 * (NW * cs + wave);
     const int tiles = (batch + 15) / 16;
-    const int b0 = 16 * (rg * tiles / groups);
-    const int lim = min(16 * ((rg + 1) * tiles / groups), batch) - 1;  // this group's last row
+    // tiles / groups tiles each, and one more in the first tiles mod groups
+    // (rg * tiles passes 2^31 from 2.1 M rows of one head on)
+    const int per = tiles / groups, extra = tiles - per * groups;
+    const int b0 = 16 * (rg * per + min(rg, extra));
+    const int lim = min(b0 + 16 * (per + (rg < extra)), batch) - 1;  // this group's last row
     // row i of A tile jt is column 8 (i / 4) + 4 jt + i mod 4 of the wave's 32,
     // so that a lane ends up with 8 adjacent columns
     E8 a[2][kLatent / 32];

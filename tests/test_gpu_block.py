@@ -90,6 +90,21 @@ def test_project_output_wide(dtype, tol, b, n_h, d_model):
     test_project_output(dtype, tol, b, n_h, d_model)
 
 
+# Rows whose tile index times the group count passes 2^31 (one head, 2.1 M rows
+# on): the output projection is the identity, so that out is the value
+# projection rounded to fp16 twice; float32 sums of 512 products.
+def test_value_projection_many_rows():
+    b = 2_200_007
+    print(f"project B={b} n_h=1", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(17)
+    o = torch.randn((b, 1, 512), generator=gen, device="cuda", dtype=torch.float16)
+    wuv, _ = _rand((1, 128, 512), 18, 512 ** -0.5, torch.float16)
+    got = capi.project_output(o, wuv, torch.eye(128, dtype=torch.float16, device="cuda"))
+    for r0 in range(0, b, 1 << 18):
+        want = o[r0:r0 + (1 << 18), 0].float() @ wuv[0].float().t()
+        torch.testing.assert_close(got[r0:r0 + (1 << 18)].float(), want, atol=1e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("n_h", [16, 128])
 def test_decode_block_equals_unabsorbed_attention(n_h):
     # absorb -> batched decode -> project, against per-head attention with
