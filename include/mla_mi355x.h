@@ -173,8 +173,10 @@ size_t mla_decode_fused_workspace_size(int num_heads, int seq_length,
                                        int num_splits);
 
 /* fp32 decode: query [num_heads x head_dim_c] fp32, cache
- * [seq_length x head_dim_c] fp32 -> out [num_heads x 512] fp32, fp32
- * products. head_dim_c must be 576. Replaces run_mla_decode_fused
+ * [seq_length x head_dim_c] fp32 -> out [num_heads x 512] fp32, products
+ * of fp32 precision: chunks of 64 tokens or more multiply operands split in two
+ * fp16 parts (22 bits) with fp32 sums where the cache's values allow it, others
+ * run on fp32 MFMAs. head_dim_c must be 576. Replaces run_mla_decode_fused
  * (csrc/mla_decode.hpp:17-22; csrc/mla_decode_fused_fwd_sm89.cu:6-60), which
  * needed num_heads % 16 == 0 and seq_length % 16 == 0 and no workspace. */
 int mla_decode_fused_fp32(const float *query, const float *cache, float *out,
@@ -312,7 +314,7 @@ int mla_decode_split_batched_fp8(const void *query, const void *cache_fp8,
  *   (the per-head values, then the output projection's fp32 K-part sums).
  * All three products are MFMA kernels of this library (fp32 accumulation)
  * and allocate nothing: W_UK and W_UV one workgroup per (head, column
- * slice), W_O streamed once from HBM through an LDS ring by at most one
+ * slice, row group), W_O streamed from HBM through an LDS ring by at most one
  * workgroup per CU, in K-parts whose fp32 sums a second small kernel adds. */
 size_t mla_project_output_workspace_size(int batch, int num_heads, int d_model);
 int mla_absorb_query_fp16(const void *q_nope, const void *q_rope,
