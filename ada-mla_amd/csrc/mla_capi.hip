@@ -58,10 +58,10 @@ constexpr int kMinSplitTokensF32 = 32;
 
 // fp32 path: 32-head workgroups once their chunks hold this many tokens (8
 // blocks). Measured per call on one box (16 / 32 heads per workgroup, one
-// workgroup per CU): n_h = 128, N = 4096 (64-token chunks at 32 heads) 20.8 /
-// 23.7 us, N = 8192 (128) 29.4 / 27.7, N = 12288 (192) 36.6 / 30.8, N = 20011
-// 53.8 / 42.1; n_h = 64, N = 9290 (146) 22.2 / 22.7, N = 32768 44.8 / 36.3;
-// n_h = 32, N = 16384 (64) 19.2 / 20.7.
+// workgroup per CU): n_h = 128, N = 4096 (64-token chunks at 32 heads) 21.5 /
+// 24.5 us, N = 6000 (96) 26.6 / 27.8, N = 8192 (128) 31.8 / 30.1, N = 12288
+// (192) 40.1 / 34.5; n_h = 64, N = 9290 (146) 24.3 / 24.5, N = 16384 (256) 30.1 /
+// 27.6; n_h = 32, N = 16384 (64) 20.7 / 22.0, N = 32768 (128) 31.0 / 29.2.
 constexpr int kHt32MinChunkTokensF32 = 128;
 
 constexpr size_t kAlign = 256;

@@ -1,6 +1,6 @@
 // fp32 split-KV MLA decode for gfx950 (the --fp32 path): same math and the
 // same partial tile layout as the fp16 kernel, with O kept unnormalised in
-// fp32, on fp32 MFMAs (16x16x4f32) or on fp16 ones over operands split in two
+// fp32, on fp32 MFMAs (16x16x4f32) or on bf16 ones over operands split in three
 // ("Products" below), so that the result keeps fp32 precision end to end.
 //
 // Replaces mla_decode_fused (reference csrc/mla_decode_fused_fwd.cuh:50-352,
@@ -41,17 +41,22 @@
 //    O waves' token-row reads (16 chunks of one row) both touch 16 distinct
 //    chunk positions of a 256-byte bank period.
 //
-// Products (kTrySplit, pieces of 4 blocks or more): fp32 MFMAs issue one
-// 16x16x4 per 32 cycles and SIMD, which bound the step (2176 cycles of them at
-// 16 heads, 4352 at 32). Both operands of both products are instead split into
-// two fp16 parts after their LDS read (22 bits, split_fp16) and three of the
-// four partial products run on 16x16x32 fp16 MFMAs with fp32 sums: 960 cycles
-// of them at 32 heads. What bounds a step then is its chain of LDS reads,
-// splits and two barriers (about 2700 cycles at 16 heads, 3300 at 32). Error
-// against float64 for N(0, 1) inputs, fp32 MFMAs -> split: 4.7e-7 -> 3.3e-7
-// (N = 4096, relative 2-norm), 3.7e-7 -> 2.6e-7 (N = 20011), 3.3e-7 -> 2.2e-7
-// (N = 65536). us per call at 128 heads, same box: N = 4096 22.7 -> 20.5,
-// N = 20011 60.0 -> 39.1, N = 65536 168.5 -> 100.5.
+// Products (kSplit, calls whose chunks hold 64 tokens or more): fp32 MFMAs issue
+// one 16x16x4 per 32 cycles and SIMD, which bound the step (2176 cycles of them
+// at 16 heads, 4352 at 32). Both operands of both products are instead split
+// into three bf16 parts after their LDS read (all 24 bits, split_bf16), and six
+// of the nine partial products run on 16x16x32 bf16 MFMAs with fp32 sums: 816
+// cycles of them at 16 heads, 1632 at 32. A step then takes 2760 cycles at 16
+// heads (3250 on fp32 MFMAs) and 4040 at 32 (5690): before barrier X the S
+// waves' chain of LDS reads, splits and MFMAs (2030 of them at 32 heads), after it the
+// O waves' second half and their wait for the next block's loads. Error against
+// float64 for N(0, 1) inputs, fp32 MFMAs -> split: 4.8e-7 -> 2.9e-7 (N = 4096,
+// relative 2-norm), 3.2e-7 -> 2.2e-7 (N = 20011), 2.5e-7 -> 2.0e-7 (N = 65536); in
+// any single value column, however small, at most 1e-6. us per call at 128
+// heads, same box: N = 4096 22.5 -> 21.0, N = 8192 35.4 -> 29.9, N = 20011
+// 60.8 -> 47.4, N = 65536 167.3 -> 127.1. (Two fp16 parts and three products were
+// faster, 20.4, 27.3, 40.0 and 101.0, but hold 22 bits of an entry and nothing
+// below 2^-36, whatever the size of its column.)
 #include <type_traits>
 
 #include "mla_device.hpp"
@@ -119,65 +124,86 @@ __device__ __forceinline__ int tile_at(int row, int chunk)
 static_assert(kRowChunks % 16 == 0, "the row swizzle stays within a row");
 static_assert(kLoads == 36, "block loads");
 
-// ---- products on fp16 MFMAs (the kernel's kSplit path): x = hi + lo / 2^11
-// with hi = fp16(x) and lo = fp16(2^11 (x - hi)), both rounded to nearest, so
-// that hi and lo hold 22 bits of x, or x to 2^-36 where that is more. Three
-// of the four partial products (hi hi, lo hi, hi lo) on fp16 MFMAs with fp32
-// sums take 3/16 of the matrix-core cycles of the fp32 product. lo is scaled
-// so that it stays a normal fp16 number as long as hi is one.
-constexpr float kLoScale = 2048.f;
-__device__ __forceinline__ void split_fp16(floatx4 x, half4 &hi, half4 &lo)
+// ---- products on bf16 MFMAs (the kernel's kSplit path): a number is the sum of
+// three bf16 parts of 8 bits, which hold all 24 (below 2^-110, where the third
+// is subnormal, what is above 2^-133), and a product the six of its nine
+// partial products that exceed 2^-24 of it, summed in fp32. This is the
+// splitting that Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", 2019) describe. bf16
+// has the exponents of fp32, so nothing depends on the values' range, and
+// subnormal operands and products are kept (both measured on gfx950).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+struct Parts4 {
+    bf16x4 p[3];
+};
+// upper 16 bits of two floats
+__device__ __forceinline__ unsigned upper_halves(float x0, float x1)
 {
-    typedef float floatx2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-    for (int i = 0; i < 4; i += 2) {
-        const half2v h = __builtin_convertvector(floatx2{x[i], x[i + 1]}, half2v);
-        const floatx2 r = {__builtin_fmaf((float)h[0], -kLoScale, x[i] * kLoScale),
-                           __builtin_fmaf((float)h[1], -kLoScale, x[i + 1] * kLoScale)};
-        const half2v l = __builtin_convertvector(r, half2v);
-        hi[i] = h[0];
-        hi[i + 1] = h[1];
-        lo[i] = l[0];
-        lo[i + 1] = l[1];
-    }
+    return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
 }
-__device__ __forceinline__ half8 join(half4 a, half4 b)
+__device__ __forceinline__ bf16x4 parts_of(unsigned lo, unsigned hi)
+{
+    return __builtin_bit_cast(bf16x4, uint2{lo, hi});
+}
+// x less the lower (upper) of two bf16 numbers, exact where the difference is:
+// one v_dot2c_f32_bf16 with (-1, 0) or (0, -1). The factors are in registers
+// the compiler cannot see into: as the inline constant -1.0, which it makes of
+// the lower one, the instruction took it for the upper number (gfx950).
+// Checked there to be exact for 2^21 random fp32 numbers of all exponents,
+// subnormal ones among them.
+struct MinusOne {
+    unsigned lower = 0x0000bf80u, upper = 0xbf800000u;
+    __device__ __forceinline__ MinusOne() { asm("" : "+s"(lower), "+s"(upper)); }
+};
+__device__ __forceinline__ float less_bf16(float x, unsigned pair, unsigned factors)
+{
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, factors), x,
+                                           false);
+}
+// The first part is x rounded or truncated, the second the rest rounded and the
+// third, exactly, what is left. The entries of C are truncated, so that those
+// up to the largest fp32 number stay finite, Q* and P rounded: the three
+// products left out are then below 2^-24 of the whole. Rounding would take the
+// largest fp32 numbers to infinity: Q*'s first parts stop at the largest bf16
+// number (kRoundFinite), P, at most 1, has none.
+constexpr float kMaxBf16 = 0x1.fep127f;
+enum FirstPart { kTruncate, kRound, kRoundFinite };
+template <FirstPart kFirst>
+__device__ __forceinline__ Parts4 split_bf16(floatx4 x, const MinusOne &m)
+{
+    unsigned w[3][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const floatx2 v = {x[2 * i], x[2 * i + 1]};
+        if constexpr (kFirst == kTruncate) {
+            w[0][i] = upper_halves(v[0], v[1]);
+        } else {
+            floatx2 f = v;
+            if constexpr (kFirst == kRoundFinite)
+                f = {__builtin_amdgcn_fmed3f(v[0], -kMaxBf16, kMaxBf16),
+                     __builtin_amdgcn_fmed3f(v[1], -kMaxBf16, kMaxBf16)};
+            w[0][i] = __builtin_bit_cast(unsigned, __builtin_convertvector(f, bf16x2));
+        }
+        const floatx2 r = {less_bf16(v[0], w[0][i], m.lower), less_bf16(v[1], w[0][i], m.upper)};
+        w[1][i] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+        w[2][i] = upper_halves(less_bf16(r[0], w[1][i], m.lower), less_bf16(r[1], w[1][i], m.upper));
+    }
+    return {parts_of(w[0][0], w[0][1]), parts_of(w[1][0], w[1][1]), parts_of(w[2][0], w[2][1])};
+}
+__device__ __forceinline__ bf16x8 join(bf16x4 a, bf16x4 b)
 {
     return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
-__device__ __forceinline__ float max_abs4(float m, floatx4 x)
-{
-    m = fmaxf(fmaxf(m, fabsf(x[0])), fabsf(x[1]));
-    return fmaxf(fmaxf(m, fabsf(x[2])), fabsf(x[3]));
-}
-// max over the wave
-__device__ __forceinline__ float wave_max(float v)
-{
-    v = max_over_lane_groups(v);
-#pragma unroll
-    for (int d = 1; d < 16; d *= 2)
-        v = fmaxf(v, __shfl_xor(v, d));
-    return v;
-}
-// The split is used while the largest entry of C lies between these: below,
-// its 2^-36 is no longer below half an fp32 ulp of that entry; above
-// (infinities included), hi overflows. The piece's first block decides the
-// path (up to kSplitMaxFirst, which leaves later blocks room to grow); a
-// piece whose later blocks pass kSplitMax is run again on fp32 MFMAs.
-constexpr float kSplitMin = 0x1p-10f;
-constexpr float kSplitMaxFirst = 0x1p12f;
-constexpr float kSplitMax = 0x1p15f;
-// P = 2^(s - m) is taken against a reference m that leaves a block's largest
-// P at 2^10 when it is set, and moves only when P would pass 2^15, so that
-// most blocks rescale nothing; P's fp16 parts then hold it to 2^-35 of that.
-constexpr float kPTop = 10.f;
-constexpr float kPMax = 15.f;
+// kSplit: a new reference max is set this far above the block's (log2 units), so
+// that P stays at most 1 and most later blocks rescale nothing.
+constexpr float kAbove = 4.f;
 
 // HT: heads per workgroup (16 or 32), as HT / 16 sub-tiles of 16 heads that
 // every wave carries side by side: the S waves' C rows and the O waves' C_N
 // columns are read from LDS once for all of them, so a 32-head workgroup
 // fills each C block once for twice the heads.
-template <int HT, bool kTrySplit>
+template <int HT, bool kSplit>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(2, 2)))
 void splitkv_fp32_kernel(const float *__restrict__ q,
                          const float *__restrict__ c,
@@ -195,20 +221,19 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
     // phase; after X they hide the softmax. 32-head tiles run all four after
     // X; 16-head tiles measure the same with one quad before it.
     constexpr int kQuadsA = kNS == 1 ? 1 : 0;
-    // kSplit: both 64-dim halves before X (N = 65536, 128 heads, with 0 / 1 / 2
-    // of them there: 105.5 / 105.7 / 102.9 us)
-    constexpr int kHalvesA = 2;
+    // kSplit: one of two 64-dim halves before X (N = 20011, 128 heads, with 0 / 1 /
+    // 2 of them there: 49.2 / 47.4 / 48.1 us; N = 4096 22.5 / 21.6 / 22.6)
+    constexpr int kHalvesA = 1;
     __shared__ __attribute__((aligned(1024))) float s_c[kRing * kSlot];
     __shared__ __attribute__((aligned(16))) float s_s[4 * HT * kTRow];
-    // P of two blocks: fp32 [head][token] tiles, or per sub-tile the lanes'
-    // fp16 parts (64 x 16 bytes [hi, hi / 2^11], then 64 x 8 bytes [lo])
-    constexpr int kPBytes = kTrySplit ? kNS * 1536 : HT * kTRow * 4;
+    // P of two blocks: fp32 [head][token] tiles, or (kSplit) per sub-tile the
+    // lanes' bf16 parts (64 x 16 bytes [first, second], then 64 x 8 [third])
+    constexpr int kPBytes = kSplit ? kNS * 1536 : HT * kTRow * 4;
     __shared__ __attribute__((aligned(16))) char s_p_mem[2 * kPBytes];
     float *s_p = reinterpret_cast<float *>(s_p_mem);
     __shared__ float s_alpha[2 * HT];
-    __shared__ float s_cmax[4];  // largest |C| of the piece's first block, by O wave
-    __shared__ int s_over[4];    // an S wave's quarter of C passed kSplitMax
 
+    const MinusOne minus;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -295,415 +320,387 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
             issue_rows(c + (size_t)t0 * kDK, p_hi - 1 - t0, s_c + (j % kRing) * kSlot);
         };
 
-        // One attempt at the piece: products on fp16 MFMAs (kSplit) or on fp32
-        // ones. kSplit, the same on every wave: kOutFirst, the first block is
-        // out of the split's range (Q* and blocks 0 and 1 are still in their
-        // slots, which a next attempt takes as `loaded`), or kOutLater, a later one.
-        constexpr int kDone = 0, kOutFirst = 1, kOutLater = 2;
-        auto attempt = [&](auto split_c, bool loaded) -> int {
-            constexpr bool kSplit = decltype(split_c)::value;
-            // the ring and the P / alpha buffers of a previous piece are free
-            __syncthreads();
-            // Prologue: Q* of the head tile (16 heads per sub-tile, swizzled
-            // like C rows) into ring slots 2 .. 2 + kNS - 1, blocks 0 and 1
-            // into slots 0 and 1, all by direct loads. The S waves take Q*
-            // into registers (and split it) as soon as it has landed, while
-            // block 0 still may not have. Q* does not pass through the
-            // compiler's own loads: it would count them, and not the direct
-            // loads issued after them, and then wait for them inside the
-            // block loop, where its vmcnt waits would drain the ring loads of
-            // block t + 2 at every step.
-            if (!loaded) {
+        // the ring and the P / alpha buffers of a previous piece are free
+        __syncthreads();
+        // Prologue: Q* of the head tile (16 heads per sub-tile, swizzled
+        // like C rows) into ring slots 2 .. 2 + kNS - 1, blocks 0 and 1
+        // into slots 0 and 1, all by direct loads. The S waves take Q*
+        // into registers (and split it) as soon as it has landed, while
+        // block 0 still may not have. Q* does not pass through the
+        // compiler's own loads: it would count them, and not the direct
+        // loads issued after them, and then wait for them inside the
+        // block loop, where its vmcnt waits would drain the ring loads of
+        // block t + 2 at every step.
 #pragma unroll
-                for (int sh = 0; sh < kNS; ++sh)
-                    issue_rows(q + ((size_t)b * num_heads + head0 + 16 * sh) * kDK, 15, s_c + (2 + sh) * kSlot);
-                issue_block(0);
-                if (nblk > 1)
-                    issue_block(1);
-            }
+        for (int sh = 0; sh < kNS; ++sh)
+            issue_rows(q + ((size_t)b * num_heads + head0 + 16 * sh) * kDK, 15, s_c + (2 + sh) * kSlot);
+        issue_block(0);
+        if (nblk > 1)
+            issue_block(1);
+        if (nblk > 1) {
+            if (s_role) MLA_WAIT_VMCNT(2 * kLoadsS); else MLA_WAIT_VMCNT(2 * kLoadsO);
+        } else {
+            if (s_role) MLA_WAIT_VMCNT(kLoadsS); else MLA_WAIT_VMCNT(kLoadsO);
+        }
+        __syncthreads();
+        auto wait_block0 = [&]() {
             if (nblk > 1) {
-                if (s_role) MLA_WAIT_VMCNT(2 * kLoadsS); else MLA_WAIT_VMCNT(2 * kLoadsO);
-            } else {
                 if (s_role) MLA_WAIT_VMCNT(kLoadsS); else MLA_WAIT_VMCNT(kLoadsO);
+            } else {
+                MLA_WAIT_VMCNT(0);
             }
-            __syncthreads();
-            auto wait_block0 = [&]() {
-                if (nblk > 1) {
-                    if (s_role) MLA_WAIT_VMCNT(kLoadsS); else MLA_WAIT_VMCNT(kLoadsO);
+            __syncthreads();  // block 0 has landed; Q* read: slots 2 .. take blocks 2 .. from step 0 on
+        };
+        // The two roles run separate loops with the same barriers (two per
+        // step), so that the S waves' Q* and the O waves' accumulators share
+        // registers.
+        if (s_role) {
+            // Q* slices, head head0 + 16 sh + l16, dims kKQ*w4 + 16*kq + 4*g .. +3
+            floatx4 qf[kNS][kSplit ? 1 : kKQ / 16];
+            // kSplit: the slice's bf16 parts; pairs of kq are one K = 32 operand,
+            // and the ninth, with two parts of C in the K of its operand, is
+            // [first, first], [second, second] and [third, first]
+            bf16x8 qp[kNS][3][kSplit ? 5 : 1];
+#pragma unroll
+            for (int sh = 0; sh < kNS; ++sh) {
+                const float *qs = s_c + (2 + sh) * kSlot;
+                floatx4 v[kKQ / 16];
+#pragma unroll
+                for (int kq = 0; kq < kKQ / 16; ++kq)
+                    v[kq] = *(const floatx4 *)(qs + slot_at(l16, 36 * w4 + 4 * kq + g));
+                if constexpr (kSplit) {
+#pragma unroll
+                    for (int pr = 0; pr < 4; ++pr) {
+                        const Parts4 a = split_bf16<kRoundFinite>(v[2 * pr], minus);
+                        const Parts4 a4 = split_bf16<kRoundFinite>(v[2 * pr + 1], minus);
+#pragma unroll
+                        for (int e = 0; e < 3; ++e)
+                            qp[sh][e][pr] = join(a.p[e], a4.p[e]);
+                    }
+                    const Parts4 a = split_bf16<kRoundFinite>(v[8], minus);
+                    qp[sh][0][4] = join(a.p[0], a.p[0]);
+                    qp[sh][1][4] = join(a.p[1], a.p[1]);
+                    qp[sh][2][4] = join(a.p[2], a.p[0]);
+                } else {
+#pragma unroll
+                    for (int kq = 0; kq < kKQ / 16; ++kq)
+                        qf[sh][kq] = v[kq];
+                }
+            }
+            wait_block0();
+            MLA_STAMP32(1, __builtin_amdgcn_s_memrealtime());
+            MLA_STAMP32(11, nblk);
+
+            float m_run = -INFINITY, l_run = 0.f;  // sub-tile my_sh; kSplit: the reference m
+            for (int t = 0; t <= nblk; ++t) {
+#ifdef MLA_TIMELINE
+                tm = MLA_MT32();
+#endif
+                if (t < nblk) {
+                    // ---- partial S^T of block t over this wave's K-quarter
+                    const float *cs = s_c + (t % kRing) * kSlot;
+                    floatx4 acc[kNS];
+                    auto row = [&](int kq) { return *(const floatx4 *)(cs + slot_at(l16, 36 * w4 + 4 * kq + g)); };
+#pragma unroll
+                    for (int sh = 0; sh < kNS; ++sh)
+                        acc[sh] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    if constexpr (kSplit) {
+                        // the products of the first parts in acc, those 2^-8
+                        // and 2^-16 as large in sums of their own
+                        floatx4 acc1[kNS], acc2[kNS];
+#pragma unroll
+                        for (int sh = 0; sh < kNS; ++sh)
+                            acc1[sh] = acc2[sh] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int pr = 0; pr < 4; ++pr) {
+                            const Parts4 a = split_bf16<kTruncate>(row(2 * pr), minus);
+                            const Parts4 a4 = split_bf16<kTruncate>(row(2 * pr + 1), minus);
+                            bf16x8 cp[3];
+#pragma unroll
+                            for (int e = 0; e < 3; ++e)
+                                cp[e] = join(a.p[e], a4.p[e]);
+#pragma unroll
+                            for (int sh = 0; sh < kNS; ++sh) {
+                                acc[sh] = mfma16x16x32(cp[0], qp[sh][0][pr], acc[sh]);
+                                acc1[sh] = mfma16x16x32(cp[0], qp[sh][1][pr], acc1[sh]);
+                                acc2[sh] = mfma16x16x32(cp[0], qp[sh][2][pr], acc2[sh]);
+                            }
+#pragma unroll
+                            for (int sh = 0; sh < kNS; ++sh) {
+                                acc1[sh] = mfma16x16x32(cp[1], qp[sh][0][pr], acc1[sh]);
+                                acc2[sh] = mfma16x16x32(cp[1], qp[sh][1][pr], acc2[sh]);
+                            }
+#pragma unroll
+                            for (int sh = 0; sh < kNS; ++sh)
+                                acc2[sh] = mfma16x16x32(cp[2], qp[sh][0][pr], acc2[sh]);
+                        }
+                        const Parts4 a = split_bf16<kTruncate>(row(8), minus);
+                        const bf16x8 c01 = join(a.p[0], a.p[1]), c02 = join(a.p[0], a.p[2]);
+                        float total = 0.f;
+#pragma unroll
+                        for (int sh = 0; sh < kNS; ++sh) {
+                            acc[sh] = mfma16x16x32(c01, qp[sh][0][4], acc[sh]);
+                            acc1[sh] = mfma16x16x32(c01, qp[sh][1][4], acc1[sh]);
+                            acc2[sh] = mfma16x16x32(c02, qp[sh][2][4], acc2[sh]);
+                        }
+#pragma unroll
+                        for (int sh = 0; sh < kNS; ++sh) {
+                            acc[sh] += acc1[sh] + acc2[sh];
+                            total += (acc[sh][0] + acc[sh][1]) + (acc[sh][2] + acc[sh][3]);
+                        }
+                        const bool lost = !(fabsf(total) < INFINITY);
+                        // the parts of an infinity make every product NaN, and
+                        // a first part's product may pass the largest number
+                        // before the others come off it. The logit itself may be
+                        // -inf, a token of no weight: the block again, on
+                        // fp32 MFMAs over Q* added up from its parts
+                        if (__builtin_expect(__builtin_amdgcn_ballot_w64(lost) != 0, 0)) {
+#pragma unroll
+                            for (int sh = 0; sh < kNS; ++sh)
+                                acc[sh] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                            for (int kq = 0; kq < kKQ / 16; ++kq) {
+                                const floatx4 x = row(kq);
+#pragma unroll
+                                for (int sh = 0; sh < kNS; ++sh) {
+                                    bf16x8 e[3] = {qp[sh][0][kq / 2], qp[sh][1][kq / 2], qp[sh][2][kq / 2]};
+                                    // (keeps the sums out of the block loop's registers)
+                                    asm volatile("" : "+v"(e[0]), "+v"(e[1]), "+v"(e[2]));
+#pragma unroll
+                                    for (int jj = 0; jj < 4; ++jj) {
+                                        const int i = 4 * (kq & 1) + jj;
+                                        acc[sh] = mfma16x16x4f32(
+                                            x[jj], ((float)e[2][i] + (float)e[1][i]) + (float)e[0][i], acc[sh]);
+                                    }
+                                }
+                            }
+                        }
+                    } else {
+#pragma unroll
+                        for (int kq = 0; kq < kKQ / 16; ++kq) {
+                            const floatx4 a = row(kq);
+#pragma unroll
+                            for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+                                for (int sh = 0; sh < kNS; ++sh)
+                                    acc[sh] = mfma16x16x4f32(a[jj], qf[sh][kq][jj], acc[sh]);
+                        }
+                    }
+#pragma unroll
+                    for (int sh = 0; sh < kNS; ++sh)
+                        *(floatx4 *)(s_s + tile_at(w4 * HT + 16 * sh + l16, g)) = acc[sh];
+                }
+#ifdef MLA_TIMELINE
+                wk_a += MLA_MT32() - tm;
+#endif
+                __syncthreads();  // barrier X: the four partial S^T tiles are in LDS
+#ifdef MLA_TIMELINE
+                { const unsigned long long t2 = MLA_MT32(); ph_a += t2 - tm; tm = t2; }
+#endif
+                if (t < nblk) {
+                    // ---- full tile and softmax of sub-tile my_sh (every S
+                    // wave of the sub-tile, identical results)
+                    const int t0 = p_lo + t * kBT;
+                    const float *sp = s_s + tile_at(16 * my_sh + l16, g);  // (the swizzle repeats every 16 rows)
+                    const floatx4 sdot = ((*(const floatx4 *)sp + *(const floatx4 *)(sp + HT * kTRow)) +
+                                          *(const floatx4 *)(sp + 2 * HT * kTRow)) +
+                                         *(const floatx4 *)(sp + 3 * HT * kTRow);
+                    float sv[4];
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        sv[i] = (t0 + 4 * g + i) < p_hi ? sdot[i] * scale_log2 : -INFINITY;
+                        mx = fmaxf(mx, sv[i]);
+                    }
+                    mx = max_over_lane_groups(mx);
+                    const float mn = !kSplit ? fmaxf(m_run, mx) : mx > m_run ? mx + kAbove : m_run;
+                    const float alpha = kSplit && mn == m_run ? 1.f : fast_exp2(m_run - mn);
+                    m_run = mn;
+                    floatx4 pv;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        pv[i] = fast_exp2(sv[i] - mn);
+                    l_run = l_run * alpha + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
+                    if (w4 < kNS) {
+                        if constexpr (kSplit) {
+                            // P's parts of tokens 4g .. +3 of head l16, as lane
+                            // (l16, g) of an O wave takes them
+                            const Parts4 pp = split_bf16<kRound>(pv, minus);
+                            char *pw = s_p_mem + (t & 1) * kPBytes + my_sh * 1536;
+                            *(bf16x8 *)(pw + 16 * lane) = join(pp.p[0], pp.p[1]);
+                            *(bf16x4 *)(pw + 1024 + 8 * lane) = pp.p[2];
+                        } else {
+                            // token 4g + i is element g of chunk i (quad-transposed)
+                            float *pw = s_p + (t & 1) * HT * kTRow;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                pw[tile_at(16 * my_sh + l16, i) + g] = pv[i];
+                        }
+                        if (g == 0)
+                            s_alpha[(t & 1) * HT + 16 * my_sh + l16] = alpha;
+                    }
+                }
+                // the S waves' share of block t + 2; block t + 1 landed before
+                // the barrier (block t + 2's loads stay in flight)
+                if (t + 2 < nblk) {
+                    issue_block(t + 2);
+                    MLA_WAIT_VMCNT(kLoadsS);
                 } else {
                     MLA_WAIT_VMCNT(0);
                 }
-                __syncthreads();  // block 0 has landed; Q* read: slots 2 .. take blocks 2 .. from step 0 on
-            };
-            // after barrier X of step 0 (kSplit): is the first block in range?
-            auto first_in_range = [&]() -> bool {
-                const float m = fmaxf(fmaxf(s_cmax[0], s_cmax[1]), fmaxf(s_cmax[2], s_cmax[3]));
-                return __builtin_amdgcn_readfirstlane(m >= kSplitMin && m <= kSplitMaxFirst);
-            };
-            // after the last barrier (kSplit): was every block?
-            auto all_in_range = [&]() -> bool {
-                return __builtin_amdgcn_readfirstlane((s_over[0] | s_over[1] | s_over[2] | s_over[3]) == 0);
-            };
-
-            // The two roles run separate loops with the same barriers (two per
-            // step), so that the S waves' Q* and the O waves' accumulators share
-            // registers.
-            if (s_role) {
-                // Q* slices, head head0 + 16 sh + l16, dims kKQ*w4 + 16*kq + 4*g .. +3
-                floatx4 qf[kNS][kSplit ? 1 : kKQ / 16];
-                // kSplit: the slice scaled by a power of two (per head and
-                // wave) that puts its largest entry in [2^13, 2^14), in fp16
-                // parts; pairs of kq are one K = 32 operand. The ninth kq meets
-                // [hi, lo] of C: as [hi, 0] and [lo, hi] (a K = 16 MFMA between
-                // K = 32 ones on one accumulator lost its sum on gfx950)
-                half8 qh[kNS][kSplit ? 5 : 1], ql[kNS][kSplit ? 5 : 1];
-                float q_unscale[kNS];
-#pragma unroll
-                for (int sh = 0; sh < kNS; ++sh) {
-                    const float *qs = s_c + (2 + sh) * kSlot;
-                    floatx4 v[kKQ / 16];
-#pragma unroll
-                    for (int kq = 0; kq < kKQ / 16; ++kq)
-                        v[kq] = *(const floatx4 *)(qs + slot_at(l16, 36 * w4 + 4 * kq + g));
-                    if constexpr (kSplit) {
-                        float mx = 0.f;
-#pragma unroll
-                        for (int kq = 0; kq < kKQ / 16; ++kq)
-                            mx = max_abs4(mx, v[kq]);
-                        mx = max_over_lane_groups(mx);
-                        // mx in [2^(k-1), 2^k); a head of zeros or below 2^-100 keeps k = -100
-                        const int k = max((int)(__float_as_uint(mx) >> 23) - 126, -100);
-                        const float up = __uint_as_float((unsigned)(127 + 14 - k) << 23);
-                        q_unscale[sh] = __uint_as_float((unsigned)(127 - 14 + k) << 23);
-#pragma unroll
-                        for (int pr = 0; pr < 4; ++pr) {
-                            half4 h0, l0, h1, l1;
-                            split_fp16(v[2 * pr] * up, h0, l0);
-                            split_fp16(v[2 * pr + 1] * up, h1, l1);
-                            qh[sh][pr] = join(h0, h1);
-                            ql[sh][pr] = join(l0, l1);
-                        }
-                        half4 h, l;
-                        split_fp16(v[8] * up, h, l);
-                        qh[sh][4] = join(h, half4{});
-                        ql[sh][4] = join(l, h);
-                    } else {
-#pragma unroll
-                        for (int kq = 0; kq < kKQ / 16; ++kq)
-                            qf[sh][kq] = v[kq];
-                    }
-                }
-                wait_block0();
-                MLA_STAMP32(1, __builtin_amdgcn_s_memrealtime());
-                MLA_STAMP32(11, nblk);
-
-                float m_run = -INFINITY, l_run = 0.f;  // sub-tile my_sh; kSplit: the reference m
-                float c_max = 0.f;                     // kSplit: largest |C| this lane has read
-                for (int t = 0; t <= nblk; ++t) {
 #ifdef MLA_TIMELINE
-                    tm = MLA_MT32();
+                { const unsigned long long t2 = MLA_MT32(); ph_b += t2 - tm; wk_b += t2 - tm; tm = t2; }
 #endif
-                    if (t < nblk) {
-                        // ---- partial S^T of block t over this wave's K-quarter
-                        const float *cs = s_c + (t % kRing) * kSlot;
-                        floatx4 acc[kNS];
-                        auto row = [&](int kq) { return *(const floatx4 *)(cs + slot_at(l16, 36 * w4 + 4 * kq + g)); };
-#pragma unroll
-                        for (int sh = 0; sh < kNS; ++sh)
-                            acc[sh] = floatx4{0.f, 0.f, 0.f, 0.f};
-                        if constexpr (kSplit) {
-                            // hi hi in acc, the cross products (2^11 times
-                            // their value) in accx
-                            floatx4 accx[kNS];
-#pragma unroll
-                            for (int sh = 0; sh < kNS; ++sh)
-                                accx[sh] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                            for (int pr = 0; pr < 4; ++pr) {
-                                const floatx4 x0 = row(2 * pr), x1 = row(2 * pr + 1);
-                                c_max = max_abs4(max_abs4(c_max, x0), x1);
-                                half4 h0, l0, h1, l1;
-                                split_fp16(x0, h0, l0);
-                                split_fp16(x1, h1, l1);
-                                const half8 hi = join(h0, h1), lo = join(l0, l1);
-#pragma unroll
-                                for (int sh = 0; sh < kNS; ++sh) {
-                                    acc[sh] = mfma16x16x32(hi, qh[sh][pr], acc[sh]);
-                                    accx[sh] = mfma16x16x32(lo, qh[sh][pr], accx[sh]);
-                                }
-#pragma unroll
-                                for (int sh = 0; sh < kNS; ++sh)
-                                    accx[sh] = mfma16x16x32(hi, ql[sh][pr], accx[sh]);
-                            }
-                            const floatx4 x = row(8);
-                            c_max = max_abs4(c_max, x);
-                            half4 h, l;
-                            split_fp16(x, h, l);
-#pragma unroll
-                            for (int sh = 0; sh < kNS; ++sh) {
-                                acc[sh] = mfma16x16x32(join(h, l), qh[sh][4], acc[sh]);
-                                accx[sh] = mfma16x16x32(join(h, l), ql[sh][4], accx[sh]);
-                            }
-#pragma unroll
-                            for (int sh = 0; sh < kNS; ++sh)
-#pragma unroll
-                                for (int i = 0; i < 4; ++i)
-                                    acc[sh][i] = __builtin_fmaf(accx[sh][i], q_unscale[sh] / kLoScale,
-                                                                acc[sh][i] * q_unscale[sh]);
-                            if (t == 0) {
-                                const float m = wave_max(c_max);
-                                if (lane == 0)
-                                    s_cmax[w4] = m;
-                            }
-                        } else {
-#pragma unroll
-                            for (int kq = 0; kq < kKQ / 16; ++kq) {
-                                const floatx4 a = row(kq);
-#pragma unroll
-                                for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-                                    for (int sh = 0; sh < kNS; ++sh)
-                                        acc[sh] = mfma16x16x4f32(a[jj], qf[sh][kq][jj], acc[sh]);
-                            }
-                        }
-#pragma unroll
-                        for (int sh = 0; sh < kNS; ++sh)
-                            *(floatx4 *)(s_s + tile_at(w4 * HT + 16 * sh + l16, g)) = acc[sh];
-                    } else if constexpr (kSplit) {
-                        const bool over = __builtin_amdgcn_ballot_w64(c_max > kSplitMax) != 0;
-                        if (lane == 0)
-                            s_over[w4] = over;
-                    }
+                __syncthreads();  // barrier Y: P and alpha of block t, block t + 1 are in LDS
 #ifdef MLA_TIMELINE
-                    wk_a += MLA_MT32() - tm;
+                { const unsigned long long t2 = MLA_MT32(); ph_o += t2 - tm; }
 #endif
-                    __syncthreads();  // barrier X: the four partial S^T tiles are in LDS
-                    if (kSplit && t == 0 && !first_in_range())
-                        return kOutFirst;
-#ifdef MLA_TIMELINE
-                    { const unsigned long long t2 = MLA_MT32(); ph_a += t2 - tm; tm = t2; }
-#endif
-                    if (t < nblk) {
-                        // ---- full tile and softmax of sub-tile my_sh (every S
-                        // wave of the sub-tile, identical results)
-                        const int t0 = p_lo + t * kBT;
-                        const float *sp = s_s + tile_at(16 * my_sh + l16, g);  // (the swizzle repeats every 16 rows)
-                        const floatx4 sdot = ((*(const floatx4 *)sp + *(const floatx4 *)(sp + HT * kTRow)) +
-                                              *(const floatx4 *)(sp + 2 * HT * kTRow)) +
-                                             *(const floatx4 *)(sp + 3 * HT * kTRow);
-                        float sv[4];
-                        float mx = -INFINITY;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            sv[i] = (t0 + 4 * g + i) < p_hi ? sdot[i] * scale_log2 : -INFINITY;
-                            mx = fmaxf(mx, sv[i]);
-                        }
-                        mx = max_over_lane_groups(mx);
-                        const float mn = !kSplit ? fmaxf(m_run, mx) : mx - m_run > kPMax ? mx - kPTop : m_run;
-                        const float alpha = kSplit && mn == m_run ? 1.f : fast_exp2(m_run - mn);
-                        m_run = mn;
-                        floatx4 pv;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            pv[i] = fast_exp2(sv[i] - mn);
-                        l_run = l_run * alpha + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
-                        if (w4 < kNS) {
-                            if constexpr (kSplit) {
-                                // P's fp16 parts (lo not scaled) of tokens 4g .. +3 of
-                                // head l16, as lane (l16, g) of an O wave takes them
-                                half4 h, l;
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) {
-                                    h[i] = (_Float16)pv[i];
-                                    l[i] = (_Float16)(pv[i] - (float)h[i]);
-                                }
-                                char *pw = s_p_mem + (t & 1) * kPBytes + my_sh * 1536;
-                                *(half8 *)(pw + 16 * lane) = join(h, h * (_Float16)(1.f / kLoScale));
-                                *(half4 *)(pw + 1024 + 8 * lane) = l;
-                            } else {
-                                // token 4g + i is element g of chunk i (quad-transposed)
-                                float *pw = s_p + (t & 1) * HT * kTRow;
-#pragma unroll
-                                for (int i = 0; i < 4; ++i)
-                                    pw[tile_at(16 * my_sh + l16, i) + g] = pv[i];
-                            }
-                            if (g == 0)
-                                s_alpha[(t & 1) * HT + 16 * my_sh + l16] = alpha;
-                        }
-                    }
-                    // the S waves' share of block t + 2; block t + 1 landed before
-                    // the barrier (block t + 2's loads stay in flight)
-                    if (t + 2 < nblk) {
-                        issue_block(t + 2);
-                        MLA_WAIT_VMCNT(kLoadsS);
-                    } else {
-                        MLA_WAIT_VMCNT(0);
-                    }
-#ifdef MLA_TIMELINE
-                    { const unsigned long long t2 = MLA_MT32(); ph_b += t2 - tm; wk_b += t2 - tm; tm = t2; }
-#endif
-                    __syncthreads();  // barrier Y: P and alpha of block t, block t + 1 are in LDS
-#ifdef MLA_TIMELINE
-                    { const unsigned long long t2 = MLA_MT32(); ph_o += t2 - tm; }
-#endif
-                }
-                MLA_STAMP32(2, __builtin_amdgcn_s_memrealtime());
-#ifdef MLA_TIMELINE
-                MLA_STAMP32(6, ph_a);
-                MLA_STAMP32(7, ph_b);
-                MLA_STAMP32(8, ph_o);
-                MLA_STAMP32W(0, 4, wk_a);
-                MLA_STAMP32W(0, 5, wk_b);
-#endif
-                if (kSplit && !all_in_range())
-                    return kOutLater;
-                const float lsum = sum_over_lane_groups(l_run);
-                if (w4 < kNS && lane < 16) {
-                    const size_t mi = (size_t)slot * num_heads + head0 + 16 * my_sh + lane;
-                    __builtin_nontemporal_store(m_run, m_part + mi);
-                    __builtin_nontemporal_store(lsum, l_part + mi);
-                }
-            } else {
-                wait_block0();
-
-                floatx4 o[kNS][8];
-#pragma unroll
-                for (int sh = 0; sh < kNS; ++sh)
-#pragma unroll
-                    for (int dt = 0; dt < 8; ++dt)
-                        o[sh][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-                // P of block j: this lane's tokens g, g + 4, g + 8, g + 12, or
-                // (kSplit) [hi, hi / 2^11] and [lo, 0] of its tokens 4g .. +3,
-                // which meet [hi, lo] of the same 4 tokens' C as one K = 32
-                // operand: 16 tokens fill it with no product missing
-                floatx4 pq[kNS];
-                half8 ph[kNS], pl[kNS];
-                // parts [k0, k1) of block j's second product: four token quads, or
-                // (kSplit) two 64-dim halves over all 16 tokens
-                constexpr int kParts = kSplit ? 2 : 4, kPartsA = kSplit ? kHalvesA : kQuadsA;
-                auto o_parts = [&](int j, auto k0, auto k1) {
-                    const float *cs = s_c + (j % kRing) * kSlot;
-                    if constexpr (kSplit) {
-#pragma unroll
-                        for (int h = decltype(k0)::value; h < decltype(k1)::value; ++h) {
-                            floatx4 x[4];
-#pragma unroll
-                            for (int r = 0; r < 4; ++r)
-                                x[r] = *(const floatx4 *)(cs + slot_at(4 * g + r, 32 * w4 + 16 * h + l16));
-#pragma unroll
-                            for (int tt = 0; tt < 4; ++tt) {
-                                half4 hi, lo;
-                                split_fp16(floatx4{x[0][tt], x[1][tt], x[2][tt], x[3][tt]}, hi, lo);
-#pragma unroll
-                                for (int sh = 0; sh < kNS; ++sh)
-                                    o[sh][4 * h + tt] = mfma16x16x32(join(hi, lo), ph[sh], o[sh][4 * h + tt]);
-#pragma unroll
-                                for (int sh = 0; sh < kNS; ++sh)
-                                    o[sh][4 * h + tt] = mfma16x16x32(join(hi, lo), pl[sh], o[sh][4 * h + tt]);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int ks = decltype(k0)::value; ks < decltype(k1)::value; ++ks) {
-                            const int row = 4 * ks + g;
-#pragma unroll
-                            for (int h = 0; h < 2; ++h) {
-                                const floatx4 a = *(const floatx4 *)(cs + slot_at(row, 32 * w4 + 16 * h + l16));
-#pragma unroll
-                                for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-                                    for (int sh = 0; sh < kNS; ++sh)
-                                        o[sh][4 * h + tt] = mfma16x16x4f32(a[tt], pq[sh][ks], o[sh][4 * h + tt]);
-                            }
-                        }
-                    }
-                };
-                for (int t = 0; t <= nblk; ++t) {
-#ifdef MLA_TIMELINE
-                    tm = MLA_MT32();
-#endif
-                    // block t + 2 into the slot that block t - 2 left at the end
-                    // of the previous step (the O waves' share)
-                    // (kSplit: at step 0 after barrier X, as it takes a slot of Q*)
-                    if (t + 2 < nblk && !(kSplit && t == 0))
-                        issue_block(t + 2);
-                    if (t >= 1) {
-                        // ---- O^T += C_N^T P^T of block t - 1 (rescaled by its alpha first)
-#pragma unroll
-                        for (int sh = 0; sh < kNS; ++sh) {
-                            if constexpr (kSplit) {
-                                const char *pr = s_p_mem + ((t - 1) & 1) * kPBytes + sh * 1536;
-                                ph[sh] = *(const half8 *)(pr + 16 * lane);
-                                pl[sh] = join(*(const half4 *)(pr + 1024 + 8 * lane), half4{});
-                            } else {
-                                pq[sh] = *(const floatx4 *)(s_p + ((t - 1) & 1) * HT * kTRow + tile_at(16 * sh + l16, g));
-                            }
-                            const float alpha = s_alpha[((t - 1) & 1) * HT + 16 * sh + l16];
-                            if (!kSplit || __builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
-#pragma unroll
-                                for (int dt = 0; dt < 8; ++dt)
-                                    o[sh][dt] *= alpha;
-                            }
-                        }
-                        o_parts(t - 1, std::integral_constant<int, 0>{}, std::integral_constant<int, kPartsA>{});
-                    }
-#ifdef MLA_TIMELINE
-                    wk_a += MLA_MT32() - tm;
-                    tm = MLA_MT32();
-#endif
-                    __syncthreads();  // barrier X
-                    if (kSplit && t == 0) {
-                        if (!first_in_range())
-                            return kOutFirst;
-                        if (t + 2 < nblk)
-                            issue_block(t + 2);
-                    }
-                    if (t >= 1)
-                        o_parts(t - 1, std::integral_constant<int, kPartsA>{}, std::integral_constant<int, kParts>{});
-                    if (t + 2 < nblk)
-                        MLA_WAIT_VMCNT(kLoadsO);
-                    else
-                        MLA_WAIT_VMCNT(0);
-#ifdef MLA_TIMELINE
-                    wk_b += MLA_MT32() - tm;
-#endif
-                    __syncthreads();  // barrier Y
-                }
-#ifdef MLA_TIMELINE
-                MLA_STAMP32W(4, 9, wk_a);
-                MLA_STAMP32W(4, 10, wk_b);
-#endif
-                if (kSplit && !all_in_range())
-                    return kOutLater;
-                // in the MFMA accumulator order of natural 16 x 16 tiles (frag_offset):
-                // lane (head j, g) holds, over o[sh][4h .. 4h+3], dims 16g .. 16g+15 of
-                // tile 8*w4 + 4h + g of sub-tile sh, element r of o[sh][4h + t]
-                // being dim 4r + t of it; each store writes 4 runs of 256
-                // contiguous bytes. Nontemporal, as the partials are read once,
-                // by the combine (see mla_splitkv_fp16.hip)
-                float *obase = o_part + (size_t)slot * num_heads * kDV;
-#pragma unroll
-                for (int sh = 0; sh < kNS; ++sh)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const floatx4 v = {o[sh][4 * h][r], o[sh][4 * h + 1][r], o[sh][4 * h + 2][r],
-                                               o[sh][4 * h + 3][r]};
-                            __builtin_nontemporal_store(
-                                v, (floatx4 *)(obase + frag_offset(head0 + 16 * sh + l16,
-                                                                   128 * w4 + 64 * h + 16 * g + 4 * r)));
-                        }
             }
-            return kDone;
-        };
-        if constexpr (kTrySplit) {
-            if (const int out = attempt(std::true_type{}, false); out != kDone) {
-                MLA_WAIT_VMCNT(0);  // ring loads in flight; the attempt's barrier follows
-                attempt(std::false_type{}, out == kOutFirst);
+            MLA_STAMP32(2, __builtin_amdgcn_s_memrealtime());
+#ifdef MLA_TIMELINE
+            MLA_STAMP32(6, ph_a);
+            MLA_STAMP32(7, ph_b);
+            MLA_STAMP32(8, ph_o);
+            MLA_STAMP32W(0, 4, wk_a);
+            MLA_STAMP32W(0, 5, wk_b);
+#endif
+            const float lsum = sum_over_lane_groups(l_run);
+            if (w4 < kNS && lane < 16) {
+                const size_t mi = (size_t)slot * num_heads + head0 + 16 * my_sh + lane;
+                __builtin_nontemporal_store(m_run, m_part + mi);
+                __builtin_nontemporal_store(lsum, l_part + mi);
             }
         } else {
-            attempt(std::false_type{}, false);
+            wait_block0();
+
+            floatx4 o[kNS][8];
+#pragma unroll
+            for (int sh = 0; sh < kNS; ++sh)
+#pragma unroll
+                for (int dt = 0; dt < 8; ++dt)
+                    o[sh][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            // P of block j: this lane's tokens g, g + 4, g + 8, g + 12, or
+            // (kSplit) of its tokens 4g .. +3 [first, first], [second, second]
+            // and [third, first], which meet [first, second] (twice) and [first,
+            // third] of the same 4 tokens' C: 16 tokens fill the K = 32 operands
+            floatx4 pq[kNS];
+            bf16x8 pp[kNS][3];
+            // parts [k0, k1) of block j's second product: four token quads, or
+            // (kSplit) two 64-dim halves over all 16 tokens
+            constexpr int kParts = kSplit ? 2 : 4, kPartsA = kSplit ? kHalvesA : kQuadsA;
+            auto o_parts = [&](int j, auto k0, auto k1) {
+                const float *cs = s_c + (j % kRing) * kSlot;
+                if constexpr (kSplit) {
+#pragma unroll
+                    for (int h = decltype(k0)::value; h < decltype(k1)::value; ++h) {
+                        floatx4 x[4];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            x[r] = *(const floatx4 *)(cs + slot_at(4 * g + r, 32 * w4 + 16 * h + l16));
+#pragma unroll
+                        for (int tt = 0; tt < 4; ++tt) {
+                            const floatx4 xt = {x[0][tt], x[1][tt], x[2][tt], x[3][tt]};
+                            const Parts4 a = split_bf16<kTruncate>(xt, minus);
+                            const bf16x8 c01 = join(a.p[0], a.p[1]), c02 = join(a.p[0], a.p[2]);
+#pragma unroll
+                            for (int sh = 0; sh < kNS; ++sh)
+                                o[sh][4 * h + tt] = mfma16x16x32(c02, pp[sh][2], o[sh][4 * h + tt]);
+#pragma unroll
+                            for (int sh = 0; sh < kNS; ++sh)
+                                o[sh][4 * h + tt] = mfma16x16x32(c01, pp[sh][1], o[sh][4 * h + tt]);
+#pragma unroll
+                            for (int sh = 0; sh < kNS; ++sh)
+                                o[sh][4 * h + tt] = mfma16x16x32(c01, pp[sh][0], o[sh][4 * h + tt]);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int ks = decltype(k0)::value; ks < decltype(k1)::value; ++ks) {
+                        const int row = 4 * ks + g;
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const floatx4 a = *(const floatx4 *)(cs + slot_at(row, 32 * w4 + 16 * h + l16));
+#pragma unroll
+                            for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                                for (int sh = 0; sh < kNS; ++sh)
+                                    o[sh][4 * h + tt] = mfma16x16x4f32(a[tt], pq[sh][ks], o[sh][4 * h + tt]);
+                        }
+                    }
+                }
+            };
+            for (int t = 0; t <= nblk; ++t) {
+#ifdef MLA_TIMELINE
+                tm = MLA_MT32();
+#endif
+                // block t + 2 into the slot that block t - 2 left at the end
+                // of the previous step (the O waves' share)
+                if (t + 2 < nblk)
+                    issue_block(t + 2);
+                if (t >= 1) {
+                    // ---- O^T += C_N^T P^T of block t - 1 (rescaled by its alpha first)
+#pragma unroll
+                    for (int sh = 0; sh < kNS; ++sh) {
+                        if constexpr (kSplit) {
+                            const char *pr = s_p_mem + ((t - 1) & 1) * kPBytes + sh * 1536;
+                            const bf16x8 p01 = *(const bf16x8 *)(pr + 16 * lane);
+                            const bf16x4 p2 = *(const bf16x4 *)(pr + 1024 + 8 * lane);
+                            const bf16x4 p0 = __builtin_shufflevector(p01, p01, 0, 1, 2, 3);
+                            const bf16x4 p1 = __builtin_shufflevector(p01, p01, 4, 5, 6, 7);
+                            pp[sh][0] = join(p0, p0);
+                            pp[sh][1] = join(p1, p1);
+                            pp[sh][2] = join(p2, p0);
+                        } else {
+                            pq[sh] = *(const floatx4 *)(s_p + ((t - 1) & 1) * HT * kTRow + tile_at(16 * sh + l16, g));
+                        }
+                        const float alpha = s_alpha[((t - 1) & 1) * HT + 16 * sh + l16];
+                        if (!kSplit || __builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+                            for (int dt = 0; dt < 8; ++dt)
+                                o[sh][dt] *= alpha;
+                        }
+                    }
+                    o_parts(t - 1, std::integral_constant<int, 0>{}, std::integral_constant<int, kPartsA>{});
+                }
+#ifdef MLA_TIMELINE
+                wk_a += MLA_MT32() - tm;
+                tm = MLA_MT32();
+#endif
+                __syncthreads();  // barrier X
+                if (t >= 1)
+                    o_parts(t - 1, std::integral_constant<int, kPartsA>{}, std::integral_constant<int, kParts>{});
+                if (t + 2 < nblk)
+                    MLA_WAIT_VMCNT(kLoadsO);
+                else
+                    MLA_WAIT_VMCNT(0);
+#ifdef MLA_TIMELINE
+                wk_b += MLA_MT32() - tm;
+#endif
+                __syncthreads();  // barrier Y
+            }
+#ifdef MLA_TIMELINE
+            MLA_STAMP32W(4, 9, wk_a);
+            MLA_STAMP32W(4, 10, wk_b);
+#endif
+            // in the MFMA accumulator order of natural 16 x 16 tiles (frag_offset):
+            // lane (head j, g) holds, over o[sh][4h .. 4h+3], dims 16g .. 16g+15 of
+            // tile 8*w4 + 4h + g of sub-tile sh, element r of o[sh][4h + t]
+            // being dim 4r + t of it; each store writes 4 runs of 256
+            // contiguous bytes. Nontemporal, as the partials are read once,
+            // by the combine (see mla_splitkv_fp16.hip)
+            float *obase = o_part + (size_t)slot * num_heads * kDV;
+#pragma unroll
+            for (int sh = 0; sh < kNS; ++sh)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const floatx4 v = {o[sh][4 * h][r], o[sh][4 * h + 1][r], o[sh][4 * h + 2][r],
+                                           o[sh][4 * h + 3][r]};
+                        __builtin_nontemporal_store(
+                            v, (floatx4 *)(obase + frag_offset(head0 + 16 * sh + l16,
+                                                               128 * w4 + 64 * h + 16 * g + 4 * r)));
+                    }
         }
 #ifdef MLA_TIMELINE
         MLA_WAIT_VMCNT(0);
@@ -721,9 +718,10 @@ hipError_t launch_splitkv_fp32(const Problem &pb, const Plan &p, const Partials 
     if (p.head_tile != 16 && p.head_tile != 32)
         return hipErrorInvalidValue;
     const dim3 grid(grid_chunks(p) * p.n_head_tiles), block(64 * kWaves);
-        // fp16-split products from chunks of 4 blocks on; shorter ones spend more on
-    // splitting Q* than on their products (N = 1024, 32-token chunks: 13.9 us
-    // against 13.4; N = 2048, 64-token ones: 16.1 against 16.9)
+    // split products from chunks of 64 tokens on, where splitting Q* begins to pay
+    // (us per call, fp32 MFMAs / split: N = 1024, 32-token chunks 13.5 / 13.9, N =
+    // 2048, 64-token ones 16.3 / 16.1, N = 3000, 96 19.3 / 18.9; 16 heads, N =
+    // 16384, 64 17.3 / 16.9)
     const bool split = p.chunk >= 64;
     auto k = p.head_tile == 32 ? (split ? splitkv_fp32_kernel<32, true> : splitkv_fp32_kernel<32, false>)
                                : (split ? splitkv_fp32_kernel<16, true> : splitkv_fp32_kernel<16, false>);

@@ -174,9 +174,9 @@ size_t mla_decode_fused_workspace_size(int num_heads, int seq_length,
 
 /* fp32 decode: query [num_heads x head_dim_c] fp32, cache
  * [seq_length x head_dim_c] fp32 -> out [num_heads x 512] fp32, products
- * of fp32 precision: chunks of 64 tokens or more multiply operands split in two
- * fp16 parts (22 bits) with fp32 sums where the cache's values allow it, others
- * run on fp32 MFMAs. head_dim_c must be 576. Replaces run_mla_decode_fused
+ * of fp32 precision whatever the values: chunks of 64 tokens or more multiply
+ * operands split in three bf16 parts (all 24 bits; what lies below 2^-110, to
+ * 2^-133) with fp32 sums, others run on fp32 MFMAs. head_dim_c must be 576. Replaces run_mla_decode_fused
  * (csrc/mla_decode.hpp:17-22; csrc/mla_decode_fused_fwd_sm89.cu:6-60), which
  * needed num_heads % 16 == 0 and seq_length % 16 == 0 and no workspace. */
 int mla_decode_fused_fp32(const float *query, const float *cache, float *out,
