@@ -720,6 +720,29 @@ bool use_wide(int batch, int K, int N)
     return batch > 32 && (int64_t)((N + 127) / 128) * (K / 64) >= kWideMinTotalSteps;
 }
 
+// Bytes of the partial tiles of the calls of up to `batch` rows, whatever the
+// device: never fewer for more rows, so that a buffer sized for the most rows of
+// a serving loop serves all its steps. A single call's need falls where its
+// row blocks get shorter: 128 heads, d_model 5120, 256 rows in one block 38.8 MB,
+// 257 rows in two blocks of 160 27.5 MB.
+size_t out_proj_part_bytes(int batch, int K, int N)
+{
+    // out_proj_kernel: two tiles for each workgroup
+    auto narrow = [&](int rows) {
+        const int64_t steps = (int64_t)((N + kCols - 1) / kCols) * ((rows + 31) / 32) * ((K + kChunk - 1) / kChunk);
+        return (size_t)2 * std::min<int64_t>(steps, kMaxGrid) * kPartTile * 4;
+    };
+    if (!use_wide(batch, K, N))
+        return narrow(batch);
+    // out_proj_wide_kernel: one for each workgroup and unit (tile g + u), of 32 rt rows
+    auto wide = [&](int64_t row_blocks, int rt) {
+        return (size_t)(kWideMaxGrid + (N + 127) / 128 * row_blocks) * 128 * 32 * rt * 4;
+    };
+    const int blocks = (batch + 255) / 256;
+    const size_t fewer = blocks > 1 ? wide(blocks - 1, 8) : narrow(32);
+    return std::max(fewer, wide(blocks, wide_rt(batch)));
+}
+
 template <typename E, int RT>
 void launch_wide(const E *x, const E *w, E *out, float *part, int batch, int K, int N, hipStream_t s)
 {
@@ -865,17 +888,9 @@ size_t mla_project_output_workspace_size(int batch, int num_heads, int d_model)
     if (batch < 1 || num_heads < 1 || num_heads > 4096 || d_model < 1)
         return 0;
     // the value projection [B x n_h*128] (16-bit), then the output
-    // projection's fp32 partial tiles: two per workgroup of at most kMaxGrid,
-    // or one per workgroup and unit, whatever the device
+    // projection's fp32 partial tiles
     const int hv = num_heads * mla::kNope;
-    size_t part;
-    if (mla::use_wide(batch, hv, d_model)) {
-        const mla::OutProjGeom geo = mla::wide_geom(batch, hv, d_model, mla::kWideMaxGrid);
-        part = ((size_t)std::min(mla::kWideMaxGrid, geo.steps) + geo.steps / geo.chunks) * 128 * 32 * mla::wide_rt(batch) * 4;
-    } else {
-        part = (size_t)2 * mla::narrow_geom(batch, hv, d_model, mla::kMaxGrid).grid * mla::kPartTile * 4;
-    }
-    return mla::align256((size_t)batch * hv * 2) + part;
+    return mla::align256((size_t)batch * hv * 2) + mla::out_proj_part_bytes(batch, hv, d_model);
 }
 
 int mla_absorb_query_fp16(const void *q_nope, const void *q_rope, const void *w_uk, void *q_star, int batch,

@@ -311,7 +311,9 @@ int mla_decode_split_batched_fp8(const void *query, const void *cache_fp8,
  *   -> out [batch][d_model] = concat_h(o_star[:, h] W_UV[h]^T) W_O^T, with
  *   the per-head values in a caller workspace of
  *   mla_project_output_workspace_size(batch, num_heads, d_model) bytes
- *   (the per-head values, then the output projection's fp32 K-part sums).
+ *   (the per-head values, then the output projection's fp32 K-part sums;
+ *   the size never falls as the batch grows, so that a workspace for the largest
+ *   batch serves every smaller one).
  * All three products are MFMA kernels of this library (fp32 accumulation)
  * and allocate nothing: W_UK and W_UV one workgroup per (head, column
  * slice, row group), W_O streamed from HBM through an LDS ring by at most one

@@ -343,6 +343,27 @@ def test_block_projection_argument_errors():
     assert lib.mla_project_output_workspace_size(3, 16, 0) == 0
 
 
+# Both forms of the output projection (more than 32 rows of 2048 or more 128 x 64
+# steps of W_O, or not), full and ragged last columns and K chunks. A workspace
+# for the largest batch of a serving loop serves every smaller one, so the size
+# never falls, and it holds each call's own need: the values and, in the wide
+# form, a tile of a row block's 32-row steps x 128 columns for each of 256
+# workgroups and each unit.
+@pytest.mark.parametrize("n_h,d_model", [(128, 5120), (32, 4096), (128, 1000), (16, 8194), (40, 7168), (2, 65535),
+                                         (16, 1000), (3, 1000), (1, 64), (1, 131072)])
+def test_project_workspace_never_falls(n_h, d_model):
+    lib = capi.load()
+    last = 0
+    for b in range(1, 1300):
+        size = lib.mla_project_output_workspace_size(b, n_h, d_model)
+        assert size >= last, b
+        last = size
+        col_blocks, blocks = -(-d_model // 128), -(-b // 256)
+        if b > 32 and col_blocks * n_h * 2 >= 2048:
+            rows = -(-(-(-b // blocks)) // 32) * 32
+            assert size >= b * n_h * 256 + (256 + col_blocks * -(-b // rows)) * 128 * rows * 4, b
+
+
 def test_block_extension_rejects_bad_inputs():
     m = _ext()
     h = torch.float16

@@ -90,6 +90,25 @@ def test_project_output_wide(dtype, tol, b, n_h, d_model):
     test_project_output(dtype, tol, b, n_h, d_model)
 
 
+# A step of a serving loop whose workspace was sized for a larger batch, where a
+# single call's need is smaller (row blocks of 160 and 192 rows against one of 256)
+@pytest.mark.parametrize("sized_for", [256, 257, 321, 513])
+def test_project_output_in_a_larger_batch_workspace(sized_for):
+    print(f"project B=256 sized for {sized_for}", flush=True)
+    b, n_h, d_model = 256, 16, 8194
+    o, o_d = _rand((b, n_h, 512), 4, 1.0, torch.float16)
+    wuv, wuv_d = _rand((n_h, 128, 512), 5, 512 ** -0.5, torch.float16)
+    wo, wo_d = _rand((d_model, n_h * 128), 6, (n_h * 128) ** -0.5, torch.float16)
+    lib = capi.load()
+    size = lib.mla_project_output_workspace_size(sized_for, n_h, d_model)
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+    out = torch.empty((b, d_model), dtype=torch.float16, device="cuda")
+    assert lib.mla_project_output_fp16(o.data_ptr(), wuv.data_ptr(), wo.data_ptr(), out.data_ptr(), ws.data_ptr(), size,
+                                       b, n_h, d_model, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(out.double().cpu().numpy(), O.project_output(o_d, wuv_d, wo_d), atol=1e-2, rtol=1e-2)
+
+
 # Rows whose tile index times the group count passes 2^31 (one head, 2.1 M rows
 # on): the output projection is the identity, so that out is the value
 # projection rounded to fp16 twice; float32 sums of 512 products.
