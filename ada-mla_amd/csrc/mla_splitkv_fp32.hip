@@ -46,15 +46,15 @@
 // at 16 heads, 4352 at 32). Both operands of both products are instead split
 // into three bf16 parts after their LDS read (all 24 bits, split_bf16), and six
 // of the nine partial products run on 16x16x32 bf16 MFMAs with fp32 sums: 816
-// cycles of them at 16 heads, 1632 at 32. A step then takes 2760 cycles at 16
-// heads (3250 on fp32 MFMAs) and 4040 at 32 (5690): before barrier X the S
-// waves' chain of LDS reads, splits and MFMAs (2030 of them at 32 heads), after it the
-// O waves' second half and their wait for the next block's loads. Error against
+// cycles of them at 16 heads, 1632 at 32. A step then takes 2650 cycles at 16
+// heads (3250 on fp32 MFMAs) and 4070 at 32 (5690): before barrier X the S
+// waves' chain of LDS reads, splits and MFMAs (2050 of them at 32 heads), after
+// it the O waves' second half and their wait for the next block's loads. Error against
 // float64 for N(0, 1) inputs, fp32 MFMAs -> split: 4.8e-7 -> 2.9e-7 (N = 4096,
 // relative 2-norm), 3.2e-7 -> 2.2e-7 (N = 20011), 2.5e-7 -> 2.0e-7 (N = 65536); in
 // any single value column, however small, at most 1e-6. us per call at 128
-// heads, same box: N = 4096 22.5 -> 21.0, N = 8192 35.4 -> 29.9, N = 20011
-// 60.8 -> 47.4, N = 65536 167.3 -> 127.1. (Two fp16 parts and three products were
+// heads, same box: N = 4096 22.5 -> 20.8, N = 8192 35.4 -> 29.9, N = 20011
+// 61.1 -> 47.1, N = 65536 168.5 -> 126.6. (Two fp16 parts and three products were
 // faster, 20.4, 27.3, 40.0 and 101.0, but hold 22 bits of an entry and nothing
 // below 2^-36, whatever the size of its column.)
 #include <type_traits>
@@ -194,6 +194,17 @@ __device__ __forceinline__ Parts4 split_bf16(floatx4 x, const MinusOne &m)
 __device__ __forceinline__ bf16x8 join(bf16x4 a, bf16x4 b)
 {
     return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// kSplit: the token of row i of an S^T tile, bits 1 and 2 of i exchanged. Lane
+// group g then holds P of tokens split_token(4g .. 4g + 3), and neither the S
+// waves' reads of rows split_token(0 .. 15) nor the O waves' of rows
+// split_token(4g + r) conflict: a 16-byte read serves lanes 0-3 and 12-15 of one
+// 16-lane group with 4-11 of the next, whose stored chunks have to differ. (In
+// order the O waves' reads conflicted, with 4g + r and g + 4r exchanged the S
+// waves': 0.23 and 0.25 of the LDS-active cycles at N = 4096.)
+__device__ __forceinline__ int split_token(int i)
+{
+    return (i & 9) | (i & 2) << 1 | (i & 4) >> 1;
 }
 // kSplit: a new reference max is set this far above the block's (log2 units), so
 // that P stays at most 1 and most later blocks rescale nothing.
@@ -391,6 +402,7 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
             MLA_STAMP32(1, __builtin_amdgcn_s_memrealtime());
             MLA_STAMP32(11, nblk);
 
+            const int s_row = kSplit ? split_token(l16) : l16;
             float m_run = -INFINITY, l_run = 0.f;  // sub-tile my_sh; kSplit: the reference m
             for (int t = 0; t <= nblk; ++t) {
 #ifdef MLA_TIMELINE
@@ -400,7 +412,7 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
                     // ---- partial S^T of block t over this wave's K-quarter
                     const float *cs = s_c + (t % kRing) * kSlot;
                     floatx4 acc[kNS];
-                    auto row = [&](int kq) { return *(const floatx4 *)(cs + slot_at(l16, 36 * w4 + 4 * kq + g)); };
+                    auto row = [&](int kq) { return *(const floatx4 *)(cs + slot_at(s_row, 36 * w4 + 4 * kq + g)); };
 #pragma unroll
                     for (int sh = 0; sh < kNS; ++sh)
                         acc[sh] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -509,7 +521,7 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
                     float mx = -INFINITY;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        sv[i] = (t0 + 4 * g + i) < p_hi ? sdot[i] * scale_log2 : -INFINITY;
+                        sv[i] = t0 + (kSplit ? split_token(4 * g + i) : 4 * g + i) < p_hi ? sdot[i] * scale_log2 : -INFINITY;
                         mx = fmaxf(mx, sv[i]);
                     }
                     mx = max_over_lane_groups(mx);
@@ -523,8 +535,8 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
                     l_run = l_run * alpha + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
                     if (w4 < kNS) {
                         if constexpr (kSplit) {
-                            // P's parts of tokens 4g .. +3 of head l16, as lane
-                            // (l16, g) of an O wave takes them
+                            // P's parts of this lane's tokens, as lane (l16, g) of
+                            // an O wave takes them
                             const Parts4 pp = split_bf16<kRound>(pv, minus);
                             char *pw = s_p_mem + (t & 1) * kPBytes + my_sh * 1536;
                             *(bf16x8 *)(pw + 16 * lane) = join(pp.p[0], pp.p[1]);
@@ -580,9 +592,9 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
                 for (int dt = 0; dt < 8; ++dt)
                     o[sh][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
             // P of block j: this lane's tokens g, g + 4, g + 8, g + 12, or
-            // (kSplit) of its tokens 4g .. +3 [first, first], [second, second]
-            // and [third, first], which meet [first, second] (twice) and [first,
-            // third] of the same 4 tokens' C: 16 tokens fill the K = 32 operands
+            // (kSplit) [first, first], [second, second] and [third, first] of its
+            // four (split_token), which meet [first, second] (twice) and [first,
+            // third] of their C: 16 tokens fill the K = 32 operands
             floatx4 pq[kNS];
             bf16x8 pp[kNS][3];
             // parts [k0, k1) of block j's second product: four token quads, or
@@ -596,7 +608,7 @@ void splitkv_fp32_kernel(const float *__restrict__ q,
                         floatx4 x[4];
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            x[r] = *(const floatx4 *)(cs + slot_at(4 * g + r, 32 * w4 + 16 * h + l16));
+                            x[r] = *(const floatx4 *)(cs + slot_at(split_token(4 * g + r), 32 * w4 + 16 * h + l16));
 #pragma unroll
                         for (int tt = 0; tt < 4; ++tt) {
                             const floatx4 xt = {x[0][tt], x[1][tt], x[2][tt], x[3][tt]};
