@@ -444,8 +444,8 @@ __global__ __launch_bounds__(256) void reduce_units_kernel(const float *__restri
 
 // Output projection of more than 32 rows (use_wide). The 32-row units above stream W_O
 // once per 32 rows; here a unit is 128 output columns x every row (32 RT of
-// them, at most 256), so that W_O crosses once and x is re-read half as often
-// per byte of it.
+// them, at most 256), so that W_O crosses once per row block and x is re-read
+// half as often per byte of it.
 //  * Same stream-K split: the (unit, 64-column K chunk) steps, units
 //    outermost, in equal contiguous ranges, one per workgroup, at most one
 //    workgroup per CU.

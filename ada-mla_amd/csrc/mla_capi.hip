@@ -120,6 +120,8 @@ int piece_cost_tokens(int head_tile)
 // the output): the two-launch fixed cost below less the combine launch.
 constexpr double kDirectFixedUs = 7.0;
 
+constexpr int kXcds = 8;
+
 // Modelled time of one 16-bit decode call (us) for a plan, fitted to MI355X
 // measurements of this library (forced plans over head tile, split count and
 // partial precision): a fixed cost per call (two launches, the prologue, the
@@ -140,7 +142,6 @@ constexpr double kDirectFixedUs = 7.0;
 // box: n_h = 16, N = 65536 114 -> 137 splits 22.9 -> 20.3 us, N = 262144
 // 108 -> 139 splits 71.3 -> 58.5 us; n_h = 32, N = 65536 114 -> 128 splits
 // 23.1 -> 20.8 us, N = 262144 (16, 108) -> (32, 179) 71.2 -> 59.0 us.
-constexpr int kXcds = 8;
 constexpr double kStreamBytesPerUs = 7.5e6;  // n_h = 16 streams C at 7.7 TB/s in the steady state
 // Calls with cu_seqlens, fitted over 184 mixes of 2 .. 128 sequences of 0 ..
 // 16384 tokens at 16 .. 128 heads: against 0.25e-6 and 0, the charge of a
